@@ -1,0 +1,1009 @@
+// gemm.hip -- multi-token dequant-fused projections on the matrix cores:
+// y[t][r] = sum_k W[r][k] x[t][k] for packed rows and T >= 2 tokens, with the
+// accuracy of an fp32 evaluation.
+//
+// Operands.  K runs in chunks of 256 (one Q4_K / Q6_K super-block, eight
+// Q5_0 / Q8_0 blocks).  x is split as x * s = hi + lo into two f16 (11 + 11
+// significant bits, |x s - hi - lo| <= 2^-23 |x s|), s the power of two that
+// brings the token's largest magnitude of the chunk into [2^14, 2^15): no
+// value overflows, and what subnormal lo parts lose is below 2^-39 of that
+// largest value.  A weight enters as an exact f16 integer or an exact pair:
+//   Q4_K        sc * (q - 8), at most 504: one f16; the chunk's d is applied
+//               once, to the chunk's sums.  The sub-blocks' offsets 8 sc and
+//               minima m ride in two extra products per chunk, against the
+//               sub-blocks' sums of x s / 32 (hi and lo).  The codes are
+//               centred because each add to the sums rounds in proportion to
+//               them (with sc * q the error against 64 bits was 1.75e-7, above
+//               the 1.2e-7 of an fp32 evaluation)
+//   Q6_K        sc * (q - 32), 13 bits: hi = the product rounded to f16, lo =
+//               the remainder (exact); d once per chunk
+//   Q5_0, Q8_0  d * q, at most 18 bits, as hi + lo (exact: every product is
+//               a multiple of 2^-24, f16's smallest step); rows of a chunk
+//               with a |d| of 256 or more take d / 256
+// Products accumulate in fp32 over the chunk on v_mfma_f32_16x16x32_f16:
+// (x hi + x lo) against one f16, or the three products hi hi + lo hi + hi lo
+// against a pair (lo lo is below 2^-22 of the term).  No group's scale is
+// applied outside the matrix cores, so the VALU only unpacks codes.
+//
+// Lane (n, g) = (lane & 15, lane >> 4) of an MFMA holds 8 codes of row n and
+// 8 activations of token n; which eight of the chunk's 256 elements is free
+// as long as both agree, so lane g takes the bytes that are contiguous in the
+// row, and step s (0..7) takes two runs of four elements ("quads"), low and
+// high, whose codes sit in one dword (K-quants: low and high nibbles) or in
+// blocks 2g and 2g + 1.  Within a quad the element order is 0, 2, 1, 3: bytes
+// 0 and 2 of a dword become an f16 pair by one and-or with 0x6400 (1024.0).
+#include "gemv.h"
+#include "mfma.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace llhip {
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+typedef float floatx4a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ floatx4 mfma_f16(const half8v& a, const half8v& b, const floatx4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ half2v as_half2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+__device__ __forceinline__ half2v splat2(_Float16 v) { return half2v{v, v}; }
+
+// Bytes 0 and 2 (or 1 and 3) of v as f16 1024 + byte: one v_perm_b32 with the
+// filler byte 0x64.
+__device__ __forceinline__ half2v bytes02(uint32_t v) {
+  return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u));
+}
+__device__ __forceinline__ half2v bytes13(uint32_t v) {
+  return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u));
+}
+__device__ __forceinline__ half8v join8(half2v a, half2v b, half2v c, half2v d) {
+  return half8v{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+// c * s as an exact pair hi + lo (c, s f16 whose product fits 22 bits).
+__device__ __forceinline__ void exact_product(half2v c, half2v s, half2v& hi, half2v& lo) {
+  hi = c * s;
+  lo = __builtin_elementwise_fma(c, s, -hi);
+}
+
+// Rows that start on any even byte: b moves down to its dword, and the dword
+// at or below the old b + o is at the returned offset from it, `shift` bytes
+// below.  (The offset is formed from the dword base, so it never goes below
+// zero, where 32 bits would wrap.)
+__device__ __forceinline__ uint32_t dword_offset(const uint8_t*& b, uint32_t o, uint32_t& shift) {
+  const uint32_t low = (uint32_t)reinterpret_cast<uintptr_t>(b) & 3u;
+  b -= low;
+  o += low;
+  shift = o & 3u;
+  return o - shift;
+}
+// N dwords from byte b + o + shift, b + o on a dword (N + 1 are read, by
+// 16-byte loads as far as they go).
+template <int N>
+__device__ __forceinline__ void load_dwords(uint32_t (&w)[N], const uint8_t* b, uint32_t o,
+                                            uint32_t shift) {
+  const uint8_t* p = b + o;
+  uint32_t t[N + 1];
+#pragma unroll
+  for (int i = 0; i + 4 <= N + 1; i += 4) {
+    const u32x4a4 v = *reinterpret_cast<const u32x4a4*>(p + 4 * i);
+    t[i] = v.x;
+    t[i + 1] = v.y;
+    t[i + 2] = v.z;
+    t[i + 3] = v.w;
+  }
+#pragma unroll
+  for (int i = (N + 1) & ~3; i < N + 1; ++i) t[i] = *reinterpret_cast<const uint32_t*>(p + 4 * i);
+#pragma unroll
+  for (int i = 0; i < N; ++i) w[i] = __builtin_amdgcn_alignbyte(t[i + 1], t[i], shift);
+}
+
+// ------------------------------------------------------------ weights
+// kBytes: one chunk of a row.  kPair: weights come as hi + lo.  kMin: the
+// Q4_K minima product.  load(): the chunk's bytes of lane g; prepare(): its
+// scales; frag(): step s's eight weights; finish(): what the chunk's sums are
+// multiplied by.  quad(g, s, high): the chunk element a quad starts at; its
+// inverse, for quad 16 q + l: step(l), and 256 g + 8 high as lane_bytes(l) +
+// quarter_bytes(q).
+template <int TYPE>
+struct GemmW;
+
+// Quads of the types whose 256 elements are 8 groups of 32: lane g takes
+// groups 2g (low) and 2g + 1 (high), step s elements 4s .. 4s + 3 of each.
+struct QuadsByGroup {
+  static __device__ __forceinline__ int quad(int g, int s, int high) {
+    return 64 * g + 32 * high + 4 * s;
+  }
+  static __device__ __forceinline__ int step(int l) { return l & 7; }
+  static __device__ __forceinline__ int lane_bytes(int l) { return 8 * (l >> 3); }
+  static constexpr int quarter_bytes(int q) { return 256 * q; }
+};
+
+template <>
+struct GemmW<kQ4_K> : QuadsByGroup {
+  static constexpr int kBytes = 144;
+  static constexpr bool kPair = false, kMin = true, kBlocks32 = false;
+  struct Raw {
+    uint4 h, q0, q1;
+  };
+  struct Scale {
+    half2v sl, ol, sh, oh;  // sc / 16 and -72 sc of sub-blocks 2g and 2g + 1
+  };
+  struct Finish {
+    // against ChunkSums: the f16 pairs {m, m} of both sub-blocks and {m0, m1};
+    // the same of 256 sc (8 sc S = 256 sc S / 32)
+    uint32_t m0, m1, m2, c0, c1, c2;
+    float d, dm;  // d and -32 dmin
+  };
+  // the 16-byte header and qs bytes [32 g, 32 g + 32); 16-byte aligned rows
+  static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g, int) {
+    r.h = load16_aligned(b + o);
+    const uint32_t q = o + 32u * (uint32_t)g;
+    r.q0 = load16_aligned(b + q + 16);
+    r.q1 = load16_aligned(b + q + 32);
+  }
+  // get-scale-min-k4-at (llambda.lisp:4316-4336) of sub-blocks 2g, 2g + 1
+  // (both at once, in bytes 0 and 1)
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    const int shift = 8 * ((2 * g) & 3);
+    const uint32_t b0 = r.h.y >> shift, b8 = r.h.w >> shift;
+    const uint32_t sc = g >= 2 ? (b8 & 0x0F0Fu) | ((b0 >> 2) & 0x3030u) : b0 & 0x3F3Fu;
+    const half2v k1152 = splat2((_Float16)-1152.f);
+    c.sl = splat2((_Float16)((float)(sc & 0xFFu) * 0.0625f));
+    c.sh = splat2((_Float16)((float)((sc >> 8) & 0xFFu) * 0.0625f));
+    c.ol = c.sl * k1152;
+    c.oh = c.sh * k1152;
+  }
+  static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale& c, int g) {
+    const int shift = 8 * ((2 * g) & 3);
+    const uint32_t b4 = r.h.z >> shift, b8 = r.h.w >> shift;
+    const uint32_t mn = g >= 2 ? ((b8 >> 4) & 0x0F0Fu) | ((b4 >> 2) & 0x3030u) : b4 & 0x3F3Fu;
+    const half2v m0 = splat2((_Float16)(float)(mn & 0xFFu));
+    const half2v m1 = splat2((_Float16)(float)((mn >> 8) & 0xFFu));
+    const half2v k4096 = splat2((_Float16)4096.f);
+    const half2v c0 = c.sl * k4096, c1 = c.sh * k4096;
+    f.m0 = __builtin_bit_cast(uint32_t, m0);
+    f.m1 = __builtin_bit_cast(uint32_t, m1);
+    f.m2 = __builtin_bit_cast(uint32_t, half2v{m0.x, m1.x});
+    f.c0 = __builtin_bit_cast(uint32_t, c0);
+    f.c1 = __builtin_bit_cast(uint32_t, c1);
+    f.c2 = __builtin_bit_cast(uint32_t, half2v{c0.x, c1.x});
+    f.d = half_bits_to_float(r.h.x & 0xFFFFu);
+    f.dm = -32.f * half_bits_to_float(r.h.x >> 16);
+  }
+  // sc (q - 8) = (1024 + 16 q) sc / 16 - 72 sc, exact in one fma
+  static __device__ __forceinline__ void frag(half8v& hi, half8v&, const Raw& r, const Scale& c,
+                                              int s) {
+    const uint4 v = s < 4 ? r.q0 : r.q1;
+    const int i = s & 3;
+    const uint32_t w = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+    const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hg = w & 0xF0F0F0F0u;
+    hi = join8(__builtin_elementwise_fma(bytes02(lo), c.sl, c.ol),
+               __builtin_elementwise_fma(bytes13(lo), c.sl, c.ol),
+               __builtin_elementwise_fma(bytes02(hg), c.sh, c.oh),
+               __builtin_elementwise_fma(bytes13(hg), c.sh, c.oh));
+  }
+};
+
+// Element 128h + 32k + l: ql byte 64h + 32 (k & 1) + l (nibble k >> 1), qh
+// byte 32h + l (bits 2k), scale 8h + 2k + (l >> 4) (llambda.lisp:4203-4310).
+// Lane g takes h = g >> 1 and l = 16 (g & 1) .. + 15; step s = 2i + kk takes
+// l = 16 (g & 1) + 4i .. + 3 of k = kk (low) and kk + 2 (high).
+template <>
+struct GemmW<kQ6_K> {
+  static constexpr int kBytes = 210;
+  static constexpr bool kPair = true, kMin = false, kBlocks32 = false;
+  static __device__ __forceinline__ int quad(int g, int s, int high) {
+    return 128 * (g >> 1) + 32 * ((s & 1) + 2 * high) + 16 * (g & 1) + 4 * (s >> 1);
+  }
+  static __device__ __forceinline__ int step(int l) { return 2 * (l & 3) + (l >> 3); }
+  static __device__ __forceinline__ int lane_bytes(int l) { return 256 * ((l >> 2) & 1); }
+  static constexpr int quarter_bytes(int q) { return 512 * (q >> 1) + 8 * (q & 1); }
+  struct Raw {
+    uint4 la, lb, qh;
+    uint32_t s[2], d;  // scales 8h .. 8h + 7
+  };
+  struct Scale {
+    half2v sc[4];
+  };
+  struct Finish {
+    float d;
+  };
+  static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g, int) {
+    // 64 (g >> 1) + 16 (g & 1) of ql, 32 (g >> 1) + 16 (g & 1) of qh, 8 (g >> 1) of the scales
+    const uint32_t h = (uint32_t)g >> 1, e = 16u * ((uint32_t)g & 1u);
+    r.d = *reinterpret_cast<const uint16_t*>(b + o + 208);
+    uint32_t sh;
+    const uint32_t a = dword_offset(b, o, sh);
+    load_dwords(reinterpret_cast<uint32_t(&)[4]>(r.la), b, a + 64 * h + e, sh);
+    load_dwords(reinterpret_cast<uint32_t(&)[4]>(r.lb), b, a + 64 * h + 32 + e, sh);
+    load_dwords(reinterpret_cast<uint32_t(&)[4]>(r.qh), b, a + 128 + 32 * h + e, sh);
+    load_dwords(r.s, b, a + 192 + 8 * h, sh);
+  }
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    const int b = 8 * (g & 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t v = r.s[k >> 1] >> (16 * (k & 1) + b);
+      c.sc[k] = splat2((_Float16)(float)(int)(int8_t)(v & 0xFFu));
+    }
+  }
+  static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale&, int) {
+    f.d = half_bits_to_float(r.d);
+  }
+  static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
+                                              int s) {
+    const int i = s >> 1, kk = s & 1;
+    const uint4 q = kk ? r.lb : r.la;
+    const uint32_t w = i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w;
+    const uint32_t v = i == 0 ? r.qh.x : i == 1 ? r.qh.y : i == 2 ? r.qh.z : r.qh.w;
+    const uint32_t cl = (w & 0x0F0F0F0Fu) | (((v >> (2 * kk)) & 0x03030303u) << 4);
+    const uint32_t ch = ((w >> 4) & 0x0F0F0F0Fu) | (((v >> (2 * kk + 4)) & 0x03030303u) << 4);
+    const half2v off = splat2((_Float16)-1056.f);
+    half2v h[4], l[4];
+    exact_product(bytes02(cl) + off, c.sc[kk], h[0], l[0]);
+    exact_product(bytes13(cl) + off, c.sc[kk], h[1], l[1]);
+    exact_product(bytes02(ch) + off, c.sc[kk + 2], h[2], l[2]);
+    exact_product(bytes13(ch) + off, c.sc[kk + 2], h[3], l[3]);
+    hi = join8(h[0], h[1], h[2], h[3]);
+    lo = join8(l[0], l[1], l[2], l[3]);
+  }
+};
+
+// Scales of a 32-block type: d of blocks 2g and 2g + 1, both / 256 where one
+// of the wave's is 256 or more (d q would leave f16's range).  Blocks past
+// the row's end (the last chunk of a K that 256 does not divide) count 0.
+struct BlockScale {
+  half2v sl, sh;
+  float d;
+  __device__ __forceinline__ void set(uint32_t d0, uint32_t d1, int g, int blocks) {
+    d0 = 2 * g < blocks ? d0 & 0xFFFFu : 0u;
+    d1 = 2 * g + 1 < blocks ? d1 & 0xFFFFu : 0u;
+    const bool wide = (d0 & 0x7FFFu) >= 0x5C00u || (d1 & 0x7FFFu) >= 0x5C00u;
+    sl = as_half2(d0 | (d0 << 16));
+    sh = as_half2(d1 | (d1 << 16));
+    d = 1.f;
+    if (__any(wide)) {
+      const half2v f = splat2((_Float16)(1.f / 256.f));
+      sl = sl * f;
+      sh = sh * f;
+      d = 256.f;
+    }
+  }
+};
+
+template <>
+struct GemmW<kQ8_0> : QuadsByGroup {
+  static constexpr int kBytes = 272;
+  static constexpr bool kPair = true, kMin = false, kBlocks32 = true;
+  struct Raw {
+    uint32_t w[17];  // blocks 2g and 2g + 1, 34 bytes each
+    int blocks;
+  };
+  typedef BlockScale Scale;
+  struct Finish {
+    float d;
+  };
+  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale& c, int) {
+    f.d = c.d;
+  }
+  static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g,
+                                              int blocks) {
+    uint32_t sh;
+    const uint32_t a = dword_offset(b, o + 68u * (uint32_t)g, sh);
+    load_dwords(r.w, b, a, sh);
+    r.blocks = blocks;
+  }
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    c.set(r.w[0], r.w[8] >> 16, g, r.blocks);
+  }
+  static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
+                                              int s) {
+    // block 2g's codes start at byte 2, block 2g + 1's at byte 36
+    const uint32_t a = __builtin_amdgcn_alignbyte(r.w[s + 1], r.w[s], 2) ^ 0x80808080u;
+    const uint32_t b = r.w[9 + s] ^ 0x80808080u;
+    const half2v off = splat2((_Float16)-1152.f);
+    half2v h[4], l[4];
+    exact_product(bytes02(a) + off, c.sl, h[0], l[0]);
+    exact_product(bytes13(a) + off, c.sl, h[1], l[1]);
+    exact_product(bytes02(b) + off, c.sh, h[2], l[2]);
+    exact_product(bytes13(b) + off, c.sh, h[3], l[3]);
+    hi = join8(h[0], h[1], h[2], h[3]);
+    lo = join8(l[0], l[1], l[2], l[3]);
+  }
+};
+
+template <>
+struct GemmW<kQ5_0> : QuadsByGroup {
+  static constexpr int kBytes = 176;
+  static constexpr bool kPair = true, kMin = false, kBlocks32 = true;
+  struct Raw {
+    uint32_t w[11];  // blocks 2g and 2g + 1, 22 bytes each
+    int blocks;
+  };
+  typedef BlockScale Scale;
+  struct Finish {
+    float d;
+  };
+  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale& c, int) {
+    f.d = c.d;
+  }
+  static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g,
+                                              int blocks) {
+    uint32_t sh;
+    const uint32_t a = dword_offset(b, o + 44u * (uint32_t)g, sh);
+    load_dwords(r.w, b, a, sh);
+    r.blocks = blocks;
+  }
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    c.set(r.w[0], r.w[5] >> 16, g, r.blocks);
+  }
+  // element 4s + b: nibble s >> 2 of qs byte 4 (s & 3) + b, fifth bit 4s + b of qh
+  static __device__ __forceinline__ uint32_t code(uint32_t qs, uint32_t qh, int s) {
+    const uint32_t n = s < 4 ? qs & 0x0F0F0F0Fu : (qs >> 4) & 0x0F0F0F0Fu;
+    uint32_t bits;  // bit i of the nibble to bit 8 i
+    asm("v_mul_u32_u24 %0, 0x204081, %1" : "=v"(bits) : "v"((qh >> (4 * s)) & 0xFu));
+    return n | ((bits & 0x01010101u) << 4);
+  }
+  static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
+                                              int s) {
+    const int i = s & 3;
+    // block 2g: qh at byte 2, qs at byte 6; block 2g + 1 at byte 22: qh 24, qs 28
+    const uint32_t qh = __builtin_amdgcn_alignbyte(r.w[1], r.w[0], 2);
+    const uint32_t qs = __builtin_amdgcn_alignbyte(r.w[i + 2], r.w[i + 1], 2);
+    const uint32_t a = code(qs, qh, s), b = code(r.w[7 + i], r.w[6], s);
+    const half2v off = splat2((_Float16)-1040.f);
+    half2v h[4], l[4];
+    exact_product(bytes02(a) + off, c.sl, h[0], l[0]);
+    exact_product(bytes13(a) + off, c.sl, h[1], l[1]);
+    exact_product(bytes02(b) + off, c.sh, h[2], l[2]);
+    exact_product(bytes13(b) + off, c.sh, h[3], l[3]);
+    hi = join8(h[0], h[1], h[2], h[3]);
+    lo = join8(l[0], l[1], l[2], l[3]);
+  }
+};
+
+// --------------------------------------------------------- activations
+// The chunk's scale of a token from its largest magnitude: s = 2^(14 - e),
+// e the exponent of `top`, and 1 / s; both normal floats (s stops growing at
+// 2^126, so chunks whose every value is below 2^-112 keep 2^-150 instead of
+// 22 bits).  With an infinity among the values s stays small enough that no
+// finite one overflows.
+__device__ __forceinline__ void chunk_scale(float top, float& s, float& inv) {
+  int e = (int)(__builtin_bit_cast(uint32_t, top) >> 23);
+  e = min(max(e, 15), 254);
+  s = __builtin_bit_cast(float, (uint32_t)(268 - e) << 23);
+  inv = __builtin_bit_cast(float, (uint32_t)(e - 14) << 23);
+}
+
+// Four elements in quad order as f16 hi and lo (two dwords each).
+__device__ __forceinline__ void split_quad(const floatx4& v, float s, uint2& hi, uint2& lo) {
+  const float e[4] = {v.x, v.z, v.y, v.w};
+  half4v h, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    h[i] = (_Float16)fmaf(e[i], s, 0.f);
+    l[i] = (_Float16)fmaf(e[i], s, -(float)h[i]);
+  }
+  hi = __builtin_bit_cast(uint2, h);
+  lo = __builtin_bit_cast(uint2, l);
+}
+
+// An infinite hi has no remainder (inf - inf would make it NaN).
+__device__ __forceinline__ uint32_t drop_inf(uint32_t hi, uint32_t lo) {
+  if ((hi & 0x7FFFu) == 0x7C00u) lo &= 0xFFFF0000u;
+  if ((hi & 0x7FFF0000u) == 0x7C000000u) lo &= 0x0000FFFFu;
+  return lo;
+}
+__device__ __forceinline__ bool infinite(float top) { return top == __builtin_inff(); }
+
+__device__ __forceinline__ float abs_max4(float m, const floatx4& v) {
+  return fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
+}
+
+// A Q4_K sub-block's sum of its 32 split activations over 32, in f16 parts:
+// the sum of the hi parts as a pair (an exact sum but for hi parts below 64:
+// 32 multiples of 2^-4 below 2^15), the sum of the lo parts as one.  The sum
+// of x itself in fp32 would carry the rounding of its five levels of adds.
+// A operand of lane (t, g): the pairs of sub-blocks 2g and 2g + 1, their lo
+// sums, zero.
+__device__ __forceinline__ float pair_sum(uint32_t h, float acc) {
+  return __builtin_amdgcn_fdot2(as_half2(h), splat2((_Float16)1.f), acc, false);
+}
+__device__ __forceinline__ uint32_t split_sum(float sum) {
+  const float v = sum * 0.03125f;
+  const _Float16 h = (_Float16)v;
+  const float hf = (float)h;
+  const _Float16 l = (_Float16)(fabsf(hf) == __builtin_inff() ? 0.f : v - hf);
+  return __builtin_bit_cast(uint32_t, half2v{h, l});
+}
+__device__ __forceinline__ uint16_t lo_sum(float sum) {
+  return __builtin_bit_cast(uint16_t, (_Float16)(sum * 0.03125f));
+}
+
+struct GemmArgs {
+  const uint8_t* w;
+  int64_t row_bytes;
+  int rows, K, chunks;
+  const float* x;
+  int64_t x_stride;
+  int tokens;
+  float* y;
+  int64_t y_stride;
+  int row_tiles, token_tiles;
+};
+
+// The chunk's sums into the totals: inv[i] = 1 / s of the tokens of D's rows.
+template <int TYPE>
+__device__ __forceinline__ void add_chunk(floatx4& tot, const floatx4& blk, const floatx4& inv,
+                                          const typename GemmW<TYPE>::Finish& c, const u32x4& sums) {
+  if constexpr (GemmW<TYPE>::kMin) {
+    const half8v a = __builtin_bit_cast(half8v, sums);
+    const half8v m = __builtin_bit_cast(half8v, u32x4{c.m0, c.m1, c.m2, 0u});
+    const half8v o = __builtin_bit_cast(half8v, u32x4{c.c0, c.c1, c.c2, 0u});
+    const floatx4 mn = mfma_f16(a, m, floatx4{0.f, 0.f, 0.f, 0.f});
+    const floatx4 all = mfma_f16(a, o, blk);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      tot[i] = fmaf(inv[i], fmaf(c.d, all[i], c.dm * mn[i]), tot[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tot[i] = fmaf(inv[i] * c.d, blk[i], tot[i]);
+  }
+}
+
+// --------------------------------------------------------- few tokens
+// One token tile of 16 per workgroup column; the workgroup's KW waves share
+// 16 RT rows and deal the chunks among themselves, each wave holding its
+// chunk's activations in registers (lane (t, g) loads, scales and splits the
+// 64 elements its own operand slots need: no LDS, no barrier before the
+// waves' sums meet).  Bound by reading the weights once and by unpacking them:
+// 7 tokens through Q4_K 14336 x 4096 take 15.0 us (2.2 TB/s; 186 us when each
+// four tokens read the rows again and the VALU formed the products).
+template <int TYPE, int RT, int KW>
+__global__ void __launch_bounds__(64 * KW)
+gemm_few_kernel(GemmArgs a) {
+  using W = GemmW<TYPE>;
+  __shared__ floatx4 red[KW > 1 ? KW - 1 : 1][RT][64];
+  const int lane = threadIdx.x & 63, kw = threadIdx.x >> 6;
+  const int n = lane & 15, g = lane >> 4;
+  const int row0 = blockIdx.x * 16 * RT, tok0 = blockIdx.y * 16;
+  const float* xr = a.x + (int64_t)min(tok0 + n, a.tokens - 1) * a.x_stride;
+  const uint8_t* wbase = a.w + (int64_t)row0 * a.row_bytes;
+  uint32_t woff[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+    woff[r] = (uint32_t)(min(row0 + 16 * r + n, a.rows - 1) - row0) * (uint32_t)a.row_bytes;
+  floatx4 tot[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  for (int c = kw; c < a.chunks; c += KW) {
+    const int blocks = W::kBlocks32 ? min(8, (a.K >> 5) - 8 * c) : 8;
+    floatx4 v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int k = 256 * c + W::quad(g, q >> 1, q & 1);
+      v[q] = (!W::kBlocks32 || k < a.K)
+                 ? (floatx4)*reinterpret_cast<const floatx4a4*>(xr + k)
+                 : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    typename W::Raw raw[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      W::load(raw[r], wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g, blocks);
+
+    float top = 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) top = abs_max4(top, v[q]);
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    float s, inv1;
+    chunk_scale(top, s, inv1);
+    half8v ah[8], al[8];
+    const bool special = __any(infinite(top));
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      uint2 h0, l0, h1, l1;
+      split_quad(v[2 * st], s, h0, l0);
+      split_quad(v[2 * st + 1], s, h1, l1);
+      ah[st] = __builtin_bit_cast(half8v, u32x4{h0.x, h0.y, h1.x, h1.y});
+      al[st] = __builtin_bit_cast(half8v, u32x4{l0.x, l0.y, l1.x, l1.y});
+    }
+    if (special) {
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        const u32x4 h = __builtin_bit_cast(u32x4, ah[st]);
+        u32x4 l = __builtin_bit_cast(u32x4, al[st]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l[i] = drop_inf(h[i], l[i]);
+        al[st] = __builtin_bit_cast(half8v, l);
+      }
+    }
+    u32x4 sums = {0u, 0u, 0u, 0u};
+    if constexpr (W::kMin) {
+      float h[2] = {0.f, 0.f}, l[2] = {0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        const u32x4 hv = __builtin_bit_cast(u32x4, ah[st]), lv = __builtin_bit_cast(u32x4, al[st]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          h[i >> 1] = pair_sum(hv[i], h[i >> 1]);
+          l[i >> 1] = pair_sum(lv[i], l[i >> 1]);
+        }
+      }
+      sums = u32x4{split_sum(h[0]), split_sum(h[1]),
+                   (uint32_t)lo_sum(l[0]) | ((uint32_t)lo_sum(l[1]) << 16), 0u};
+    }
+    floatx4 inv;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) inv[i] = __shfl(inv1, 4 * g + i);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      typename W::Scale sc;
+      W::prepare(sc, raw[r], g);
+      // the small products first: each add to the sums rounds in proportion
+      // to what they have reached
+      floatx4 blk = {0.f, 0.f, 0.f, 0.f};
+      half8v bh[8], bl;
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        W::frag(bh[st], bl, raw[r], sc, st);
+        blk = mfma_f16(al[st], bh[st], blk);
+        if constexpr (W::kPair) blk = mfma_f16(ah[st], bl, blk);
+      }
+#pragma unroll
+      for (int st = 0; st < 8; ++st) blk = mfma_f16(ah[st], bh[st], blk);
+      typename W::Finish fin;
+      W::finish(fin, raw[r], sc, g);
+      add_chunk<TYPE>(tot[r], blk, inv, fin, sums);
+    }
+  }
+  if constexpr (KW > 1) {
+    if (kw > 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r) red[kw - 1][r][lane] = tot[r];
+    }
+    __syncthreads();
+    // wave w adds row tiles w, w + KW, ... in wave order
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      if (kw != 0) break;
+#pragma unroll
+      for (int q = 0; q < KW - 1; ++q) tot[r] += red[q][r][lane];
+    }
+    if (kw != 0) return;
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int row = row0 + 16 * r + n;
+    if (row < a.rows)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = tok0 + 4 * g + i;
+        if (t < a.tokens) a.y[(int64_t)t * a.y_stride + row] = tot[r][i];
+      }
+  }
+}
+
+// Sums of V (4 or 8) values over aligned groups of eight lanes; lane i of a
+// group receives the sum of value i (i % 4 for V = 4).  b2, b1, b0: bits of i.
+template <int V>
+__device__ __forceinline__ float scatter_sum(const float* v, bool b2, bool b1, bool b0) {
+  float r[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (V == 8)
+      r[k] = (b2 ? v[k + 4] : v[k]) + dpp<kDppHalfMirror>(b2 ? v[k] : v[k + 4]);
+    else
+      r[k] = v[k] + dpp<kDppHalfMirror>(v[k]);
+  }
+  float u[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) u[k] = (b1 ? r[k + 2] : r[k]) + dpp<kDppXor2>(b1 ? r[k] : r[k + 2]);
+  return (b0 ? u[1] : u[0]) + dpp<kDppXor1>(b0 ? u[0] : u[1]);
+}
+
+// --------------------------------------------------------- many tokens
+// RW waves of 16 RT rows each share the split activations of 16 JT tokens in
+// LDS; KW such groups deal the chunks among themselves.  Two chunks' images
+// take turns: the next chunk's activations are requested before this chunk's
+// products and split after them, so a chunk costs one barrier and its memory
+// round trips run beside the products; the next chunk's weights go straight
+// from memory into registers.  A load instruction covers 64 elements of four
+// tokens (256 contiguous bytes each), the token's largest magnitude meets over
+// 16 lanes, and the operand image is [token tile][step][hi, lo][16 bytes per
+// lane], lane positions XORed with the step so that the writes of one
+// instruction spread over the banks.
+// Measured: 2048 tokens through Q4_K 14336 x 4096 0.67 ms (360 TFLOP/s; 49.8
+// ms before, in passes of four tokens on the VALU), 1000 tokens through Q6_K
+// 4096 x 14336 0.41 ms (31.7), 129 through Q8_0 1024 x 2688 14.9 us (517).
+// Bound by the VALU beside the MFMAs (unpacking and splitting: about four
+// instructions per MFMA, two of which issue beside it) and the operand reads
+// (a wave of 32 rows reads each split activation once per 32 rows).
+template <int TYPE, int JT>
+struct GemmLds {
+  static constexpr int kX = JT * 16384;             // split activations
+  static constexpr int kInv = kX;                   // 1 / s per token
+  static constexpr int kSums = kInv + JT * 64;      // Q4_K: the sums' operands
+  static constexpr int kBytes = kSums + (GemmW<TYPE>::kMin ? JT * 1024 : 0);
+};
+
+template <int TYPE, int RT, int JT, int RW, int KW>
+__global__ void __launch_bounds__(64 * RW * KW, 2)
+gemm_many_kernel(GemmArgs a) {
+  using W = GemmW<TYPE>;
+  using L = GemmLds<TYPE, JT>;
+  constexpr int P = 4 * JT / RW;  // groups of four tokens a wave splits
+  static_assert(P * RW == 4 * JT, "token groups");
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int rw = wave % RW, kw = wave / RW;
+  const int n = lane & 15, g = lane >> 4;
+  uint8_t* lds = smem + kw * 2 * L::kBytes;
+
+  // Workgroup b runs on XCD b % 8: each XCD takes one contiguous run of
+  // tiles, in groups of 8 row tiles by all token tiles, so that the tiles in
+  // flight on an XCD share rows and tokens in its L2.
+  const int total = a.row_tiles * a.token_tiles, per = (total + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= total || (int)(blockIdx.x >> 3) >= per) return;
+  const int band = tile / (8 * a.token_tiles), rest = tile - band * 8 * a.token_tiles;
+  const int band_rows = min(8, a.row_tiles - 8 * band);
+  const int tt = rest / band_rows, rt = 8 * band + (rest - tt * band_rows);
+  const int row0 = (rt * RW + rw) * 16 * RT, tok0 = tt * 16 * JT;
+
+  // uniform bases and 32-bit lane offsets (gemm_launch bounds the strides)
+  const int rbase = __builtin_amdgcn_readfirstlane(min(row0, a.rows - 1));
+  const uint8_t* wbase = a.w + (int64_t)rbase * a.row_bytes;
+  uint32_t woff[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+    woff[r] = (uint32_t)(min(row0 + 16 * r + n, a.rows - 1) - rbase) * (uint32_t)a.row_bytes;
+  const float* xbase = a.x + (int64_t)tok0 * a.x_stride;
+  uint32_t xoff[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+    xoff[p] = 4 * ((uint32_t)(min(tok0 + 4 * (P * rw + p) + g, a.tokens - 1) - tok0) *
+                       (uint32_t)a.x_stride + 4 * n);
+
+  floatx4 tot[RT][JT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int j = 0; j < JT; ++j) tot[r][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  typename W::Raw raw[RT];
+  auto load_rows = [&](int c) {
+    const int blocks = W::kBlocks32 ? min(8, (a.K >> 5) - 8 * c) : 8;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      W::load(raw[r], wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g, blocks);
+  };
+  // v[p][q]: token 4 (P rw + p) + g, elements 64 q + 4 n .. + 3
+  floatx4 v[P][4];
+  auto load_x = [&](int c) {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        v[p][q] = (!W::kBlocks32 || 256 * c + 64 * q + 4 * n < a.K)
+                      ? (floatx4)*reinterpret_cast<const floatx4a4*>(
+                            reinterpret_cast<const uint8_t*>(xbase + 256 * c) + (xoff[p] + 256u * q))
+                      : floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto split_x = [&](uint8_t* buf) {
+    const int own = (int)opaque((uint32_t)lane);  // addresses not kept over the products
+    const int n = own & 15, g = own >> 4;
+    float top[P], most = 0.f;
+    float hs[W::kMin ? 4 * P : 1], ls[W::kMin ? 4 * P : 1];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      float m = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) m = abs_max4(m, v[p][q]);
+      m = fmaxf(m, dpp<kDppXor1>(m));
+      m = fmaxf(m, dpp<kDppXor2>(m));
+      m = fmaxf(m, dpp<kDppHalfMirror>(m));
+      top[p] = fmaxf(m, dpp<kDppMirror>(m));
+      most = fmaxf(most, top[p]);
+    }
+    const int step = W::step(n);
+    uint8_t* lane_at = buf + 2048 * step + W::lane_bytes(n);
+    // the group's first token is token t of the workgroup's
+    auto image = [&](int t) {
+      return lane_at + 16384 * (t >> 4) + 128 * ((t >> 3) & 1) + 16 * (((t & 4) + g) ^ step);
+    };
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      float s, inv;
+      chunk_scale(top[p], s, inv);
+      const int t = 4 * (P * rw + p);
+      uint8_t* at = image(t);
+      reinterpret_cast<float*>(buf + L::kInv)[t + g] = inv;  // 16 lanes, one value
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint2 hi, lo;
+        split_quad(v[p][q], s, hi, lo);
+        *reinterpret_cast<uint2*>(at + W::quarter_bytes(q)) = hi;
+        *reinterpret_cast<uint2*>(at + W::quarter_bytes(q) + 1024) = lo;
+        if constexpr (W::kMin) {
+          hs[4 * p + q] = pair_sum(hi.y, pair_sum(hi.x, 0.f));
+          ls[4 * p + q] = pair_sum(lo.y, pair_sum(lo.x, 0.f));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (W::kMin) {
+      // sub-block 2q + (n >> 3) of token t + g: sums over eight lanes, lane n & 7
+      // taking value n & 7 of the eight (p, q) of two token groups
+      constexpr int V = 4 * P < 8 ? 4 * P : 8;
+      const bool b2 = n & 4, b1 = n & 2, b0 = n & 1;
+#pragma unroll
+      for (int at = 0; at < 4 * P; at += V) {
+        const float h = scatter_sum<V>(hs + at, b2, b1, b0), l = scatter_sum<V>(ls + at, b2, b1, b0);
+        const int i = at + (n & (V - 1)), t = 4 * (P * rw + (i >> 2));
+        uint8_t* to = buf + L::kSums + 1024 * (t >> 4) + 16 * ((t & 15) + g + 16 * (i & 3));
+        *reinterpret_cast<uint32_t*>(to + 4 * (n >> 3)) = split_sum(h);
+        *reinterpret_cast<uint16_t*>(to + 8 + 2 * (n >> 3)) = lo_sum(fabsf(h) == __builtin_inff() ? 0.f : l);
+      }
+    }
+    if (__any(infinite(most))) {
+      // an infinity has no remainder (inf - inf made it NaN)
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        uint8_t* at = image(4 * (P * rw + p)) + 1024;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (infinite(fabsf(v[p][q][e])))
+              *reinterpret_cast<uint16_t*>(at + W::quarter_bytes(q) + 4 * (e & 1) + (e & 2)) = 0;
+      }
+    }
+  };
+
+  // y = tot, or y += tot with every y requested before the first add (the
+  // addresses are formed here each time: kept over the chunks they cost the
+  // products their registers)
+  auto store_rows = [&](bool add) {
+    const int at = (int)opaque((uint32_t)lane);
+    const int left = a.rows - row0 - (at & 15), t0 = tok0 + 4 * (at >> 4);
+    float* y0 = a.y + (int64_t)t0 * a.y_stride + row0 + (at & 15);
+    auto each = [&](auto&& f) {
+      float* y = y0;
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (t0 + 16 * j + i < a.tokens) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+              if (16 * r < left) f(y[16 * r], r, j, i);
+          }
+          y += a.y_stride;
+        }
+        y += 12 * a.y_stride;
+      }
+    };
+    if (add) {
+      floatx4 was[RT][JT];
+      each([&](float& v, int r, int j, int i) { was[r][j][i] = v; });
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int j = 0; j < JT; ++j) tot[r][j] += was[r][j];
+    }
+    each([&](float& v, int r, int j, int i) { v = tot[r][j][i]; });
+  };
+  // One group's totals go out every 8 chunks and start again: each add to them
+  // rounds in proportion to what they have reached (16 chunks of Q4_K in one
+  // run: 1.24e-7 against 64 bits, an fp32 evaluation 1.17e-7)
+  constexpr int kSegment = 8;
+
+  const int iters = (a.chunks + KW - 1) / KW;
+  if (kw < a.chunks) {
+    load_rows(kw);
+    load_x(kw);
+    split_x(lds);
+  }
+  __syncthreads();
+  for (int it = 0; it < iters; ++it) {
+    const int c = it * KW + kw;
+    uint8_t* buf = lds + (it & 1) * L::kBytes;
+    if (c < a.chunks) {
+      const bool more = c + KW < a.chunks;
+      if (more) load_x(c + KW);
+      __builtin_amdgcn_sched_barrier(0);
+      typename W::Scale sc[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) W::prepare(sc[r], raw[r], g);
+      // the small products have sums of their own where registers allow: each
+      // add rounds in proportion to the sum it meets
+      constexpr bool kOwnLo = RT * JT <= 8;
+      floatx4 blk[RT][JT], low[kOwnLo ? RT : 1][kOwnLo ? JT : 1];
+      const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+      // operand i = (step i / JT, token tile i % JT), read one ahead
+      const uint32_t unit = opaque((uint32_t)lane);
+      auto operand = [&](int i, half8v& hi, half8v& lo) {
+        const int st = i / JT;
+        const uint8_t* at = buf + 16 * (unit ^ (uint32_t)st) + (i % JT) * 16384 + st * 2048;
+        hi = *reinterpret_cast<const half8v*>(at);
+        lo = *reinterpret_cast<const half8v*>(at + 1024);
+      };
+      half8v ah[2], al[2], bh[RT], bl[RT];
+      operand(0, ah[0], al[0]);
+#pragma unroll
+      for (int i = 0; i < 8 * JT; ++i) {
+        const int st = i / JT, j = i % JT;
+        if (j == 0) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) W::frag(bh[r], bl[r], raw[r], sc[r], st);
+        }
+        if (i + 1 < 8 * JT) operand(i + 1, ah[(i + 1) & 1], al[(i + 1) & 1]);
+        const half8v h = ah[i & 1], l = al[i & 1];
+        auto low_sum = [&](int r) -> floatx4& { return kOwnLo ? low[kOwnLo ? r : 0][kOwnLo ? j : 0] : blk[r][j]; };
+#pragma unroll
+        for (int r = 0; r < RT; ++r) low_sum(r) = mfma_f16(l, bh[r], st ? low_sum(r) : zero);
+        if constexpr (W::kPair)
+#pragma unroll
+          for (int r = 0; r < RT; ++r) low_sum(r) = mfma_f16(h, bl[r], low_sum(r));
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          blk[r][j] = mfma_f16(h, bh[r], kOwnLo && st == 0 ? zero : blk[r][j]);
+        if (j == JT - 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      typename W::Finish fin[RT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) W::finish(fin[r], raw[r], sc[r], g);
+      if (more) load_rows(c + KW);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+        const floatx4 inv = *reinterpret_cast<const floatx4*>(buf + L::kInv + 64 * j + 16 * g);
+        u32x4 sums = {0u, 0u, 0u, 0u};
+        if constexpr (W::kMin) {
+          sums = *reinterpret_cast<const u32x4*>(buf + L::kSums + j * 1024 + 16 * lane);
+          sums[3] = 0u;  // never written
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          if constexpr (kOwnLo) blk[r][j] += low[r][j];
+          add_chunk<TYPE>(tot[r][j], blk[r][j], inv, fin[r], sums);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (more) split_x(lds + ((it + 1) & 1) * L::kBytes);
+      if (KW == 1 && more && it % kSegment == kSegment - 1) {
+        store_rows(it >= kSegment);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int j = 0; j < JT; ++j) tot[r][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    __syncthreads();
+  }
+
+  if constexpr (KW > 1) {
+    floatx4* red = reinterpret_cast<floatx4*>(smem);  // [KW - 1][RW][RT * JT][64]
+    if (kw > 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int j = 0; j < JT; ++j)
+          red[(((kw - 1) * RW + rw) * RT * JT + r * JT + j) * 64 + lane] = tot[r][j];
+    }
+    __syncthreads();
+    if (kw > 0) return;
+#pragma unroll
+    for (int q = 0; q < KW - 1; ++q)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int j = 0; j < JT; ++j)
+          tot[r][j] += red[((q * RW + rw) * RT * JT + r * JT + j) * 64 + lane];
+  }
+  store_rows(iters > kSegment && KW == 1);
+}
+
+// ------------------------------------------------------------------ host
+template <int TYPE, int RT, int KW>
+static hipError_t launch_few(const GemmArgs& a, hipStream_t stream) {
+  const dim3 grid((a.rows + 16 * RT - 1) / (16 * RT), (a.tokens + 15) / 16);
+  if (grid.y > 65535) return hipErrorInvalidValue;  // never chosen: rounds make it the slowest
+  hipLaunchKernelGGL((gemm_few_kernel<TYPE, RT, KW>), grid, dim3(64 * KW), 0, stream, a);
+  return hipGetLastError();
+}
+
+template <int TYPE, int RT, int JT, int RW, int KW>
+static hipError_t launch_many(const GemmArgs& a_in, hipStream_t stream) {
+  GemmArgs a = a_in;
+  a.row_tiles = (a.rows + 16 * RT * RW - 1) / (16 * RT * RW);
+  a.token_tiles = (a.tokens + 16 * JT - 1) / (16 * JT);
+  const int64_t total = (int64_t)a.row_tiles * a.token_tiles;
+  if (total > (1 << 30)) return hipErrorInvalidValue;
+  constexpr int lds = KW * 2 * GemmLds<TYPE, JT>::kBytes;
+  static_assert(lds <= (int)kMaxLdsBytes && (KW - 1) * RW * RT * JT * 1024 <= lds, "LDS");
+  const auto kernel = gemm_many_kernel<TYPE, RT, JT, RW, KW>;
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * ((total + 7) / 8))), dim3(64 * RW * KW), lds,
+                     stream, a);
+  return hipGetLastError();
+}
+
+template <int TYPE>
+static hipError_t launch_type(const GemmArgs& a, bool one_order, hipStream_t stream) {
+  // one shape for every batch: the one in the middle (64 x 16)
+  if (one_order) return launch_many<TYPE, 2, 1, 2, 4>(a, stream);
+  // The tile shape whose workgroups, one to a CU, finish first: rounds of
+  // workgroups times a workgroup's time, in 0.1 us for 16 chunks of Q4_K
+  // (measured with one round; the other types' times stand in the same
+  // proportions).  Small tiles leave fewer CUs idle, large ones decode and
+  // split less per product: 256 x 64 does 172 rows x tokens a us, 128 x 32
+  // 117, 32 x 16 40.
+  struct Shape {
+    int rows, tokens, base, per_token;  // per_token: of the first 16 tokens
+  };
+  static constexpr Shape shapes[] = {
+      {64, 16, 138, 3}, {32, 16, 95, 3}, {16, 16, 77, 2},             // few
+      {32, 16, 128, 0}, {64, 16, 166, 0}, {128, 32, 350, 0},          // many
+      {128, 64, 670, 0}, {256, 64, 950, 0}};
+  const int64_t cus = device_cu_count();
+  int best = 0;
+  int64_t least = INT64_MAX;
+  for (int i = 0; i < (int)(sizeof shapes / sizeof shapes[0]); ++i) {
+    const Shape& s = shapes[i];
+    const int64_t groups = (int64_t)((a.rows + s.rows - 1) / s.rows) * ((a.tokens + s.tokens - 1) / s.tokens);
+    const int64_t time = (groups + cus - 1) / cus * (s.base + s.per_token * std::min(a.tokens, 16));
+    if (time < least) {
+      least = time;
+      best = i;
+    }
+  }
+  switch (best) {
+    case 0: return launch_few<TYPE, 4, 8>(a, stream);
+    case 1: return launch_few<TYPE, 2, 8>(a, stream);
+    case 2: return launch_few<TYPE, 1, 8>(a, stream);
+    case 3: return launch_many<TYPE, 1, 1, 2, 4>(a, stream);
+    case 4: return launch_many<TYPE, 2, 1, 2, 4>(a, stream);
+    case 5: return launch_many<TYPE, 2, 2, 4, 2>(a, stream);
+    case 6: return launch_many<TYPE, 1, 4, 8, 1>(a, stream);
+    default: return launch_many<TYPE, 2, 4, 8, 1>(a, stream);
+  }
+}
+
+hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream) {
+  if (p.tokens < 1 || p.rows < 1 || p.rows > INT32_MAX || p.columns % block_weights(p.type))
+    return hipErrorInvalidValue;
+  // 16-byte loads of Q4_K rows, dword loads at or below the other types'
+  if (reinterpret_cast<uintptr_t>(p.weights) % (p.type == kQ4_K ? 16 : 2)) return hipErrorInvalidValue;
+  // lane offsets within a tile are 32 bits
+  if (p.x_stride < 0 || p.x_stride > (1 << 22) || p.row_bytes > (1 << 22)) return hipErrorInvalidValue;
+  GemmArgs a{};
+  a.w = p.weights;
+  a.row_bytes = p.row_bytes;
+  a.rows = (int)p.rows;
+  a.K = (int)p.columns;
+  a.chunks = (a.K + 255) / 256;
+  a.x = p.x;
+  a.x_stride = p.x_stride;
+  a.tokens = p.tokens;
+  a.y = p.y;
+  a.y_stride = p.y_stride;
+  switch (p.type) {
+    case kQ4_K: return launch_type<kQ4_K>(a, p.one_order, stream);
+    case kQ6_K: return launch_type<kQ6_K>(a, p.one_order, stream);
+    case kQ5_0: return launch_type<kQ5_0>(a, p.one_order, stream);
+    case kQ8_0: return launch_type<kQ8_0>(a, p.one_order, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace llhip

@@ -19,6 +19,10 @@ struct GemvProblem {
   int tokens;
   float* y;
   int64_t y_stride;
+  // several tokens: every token's sums in one order whatever `tokens` is
+  // (equal bit for bit in any batch of two or more), at the price of one tile
+  // shape for all batches
+  bool one_order = false;
 };
 
 // LDS per workgroup on gfx950.
@@ -71,6 +75,9 @@ hipError_t gemv_fused_pair_launch(const GemvProblem& pa, const GemvFuse& fa, con
 // Batch-1 Q4_K / Q6_K GEMV on MFMA (gemv_mfma.hip).
 bool gemv_mfma_supported(const GemvProblem& p);
 hipError_t gemv_mfma_launch(const GemvProblem& p, hipStream_t stream);
+
+// Q4_K / Q6_K / Q5_0 / Q8_0 products of two or more tokens on MFMA (gemm.hip).
+hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream);
 
 // Compute units of the current device (cached after the first call).
 int device_cu_count();

@@ -4,9 +4,12 @@
 // Q5_0, Q8_0 (units.h) and F32, i.e. %gguf-model-matrix-vector-multiply-into
 // (llambda.lisp:4542-4658) on one MI355X.
 //
-// Launch shape: 256-thread workgroups (4 wavefronts).  Each workgroup copies
-// the activations of up to NT tokens into LDS once, with the sums of every
-// 16-element group, then its wavefronts stream rows: a wavefront owns
+// Several tokens of packed rows run on MFMA (gemm.hip), one token of Q4_K and
+// Q6_K too (gemv_mfma.hip); here are one token of the other rows, and F32.
+// Launch shape of rows whose K 64 does not divide: 256-thread workgroups (4
+// wavefronts).  Each workgroup copies the token's activations into LDS once,
+// with the sums of every 16-element group, then its wavefronts stream rows: a
+// wavefront owns
 // `slots` row slots of `lpr` lanes (lpr = min(64, pow2ceil(K/32))), every lane
 // dequantises one 32-weight unit per step with 16-byte loads, and the row's
 // lanes are summed with cross-lane shuffles.  R rows per slot are loaded
@@ -18,15 +21,14 @@
 
 namespace llhip {
 
-template <int TYPE, int NT, int R>
+template <int TYPE, int R>
 __global__ void __launch_bounds__(256)
 gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
-            const float* __restrict__ x, int64_t x_stride, int ntok,
-            float* __restrict__ y, int64_t y_stride, int lpr_log2) {
+            const float* __restrict__ x, float* __restrict__ y, int lpr_log2) {
   extern __shared__ float smem[];
   float* xs = smem;
-  float* xg = smem + NT * K;
-  stage_x<NT>(xs, xg, x, x_stride, ntok, K);
+  float* xg = smem + K;
+  stage_x<1>(xs, xg, x, K, 1, K);
   __syncthreads();
   const XView xv{xs, xg, K, K >> 4};
 
@@ -42,7 +44,7 @@ gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
   const int stride = gridDim.x * waves_per_block * rows_per_iter;
 
   for (int base = (blockIdx.x * waves_per_block + wave) * rows_per_iter; base < rows; base += stride) {
-    float acc[R][NT];
+    float acc[R][1];
     const uint8_t* rp[R];
     bool valid[R];
 #pragma unroll
@@ -51,15 +53,12 @@ gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
       valid[r] = row < rows;
       rp[r] = w + (int64_t)(valid[r] ? row : 0) * row_bytes;
     }
-    rows_dot<TYPE, NT, R>(rp, valid, l, lpr, units, xv, acc);
+    rows_dot<TYPE, 1, R>(rp, valid, l, lpr, units, xv, acc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int row = base + r * slots + slot;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float v = segment_sum_dyn(acc[r][t], lpr);
-        if (l == 0 && row < rows && t < ntok) y[t * y_stride + row] = v;
-      }
+      const float v = segment_sum_dyn(acc[r][0], lpr);
+      if (l == 0 && row < rows) y[row] = v;
     }
   }
 }
@@ -330,19 +329,20 @@ static hipError_t launch_with_lds(Kernel k, int grid, size_t lds, hipStream_t st
   return hipGetLastError();
 }
 
-template <int TYPE, int NT, int R>
+template <int TYPE>
 static hipError_t launch_packed(const GemvProblem& p, hipStream_t stream) {
+  constexpr int R = 2;
   const int lpr_log2 = lanes_per_row_log2((int)p.columns);
   const int slots = kWave >> lpr_log2;
   const int rows_per_block = 4 * slots * R;
   const int needed = (int)((p.rows + rows_per_block - 1) / rows_per_block);
-  const size_t lds = (size_t)NT * (p.columns + (p.columns >> 4)) * sizeof(float);
+  const size_t lds = (size_t)(p.columns + (p.columns >> 4)) * sizeof(float);
+  if (lds > kMaxLdsBytes) return hipErrorInvalidValue;
   // Enough workgroups for 8 per CU; beyond that, workgroups loop over rows so
   // the activation staging is amortised.
   const int grid = std::max(1, std::min(needed, device_cu_count() * 8));
-  return launch_with_lds(gemv_kernel<TYPE, NT, R>, grid, lds, stream, p.weights, p.row_bytes,
-                         (int)p.rows, (int)p.columns, p.x, p.x_stride, p.tokens, p.y, p.y_stride,
-                         lpr_log2);
+  return launch_with_lds(gemv_kernel<TYPE, R>, grid, lds, stream, p.weights, p.row_bytes,
+                         (int)p.rows, (int)p.columns, p.x, p.y, lpr_log2);
 }
 
 template <int NT>
@@ -353,18 +353,6 @@ static hipError_t launch_f32(const GemvProblem& p, hipStream_t stream) {
   return launch_with_lds(gemv_f32_kernel<NT>, grid, lds, stream,
                          reinterpret_cast<const float*>(p.weights), (int)p.rows, (int)p.columns,
                          p.x, p.x_stride, p.tokens, p.y, p.y_stride);
-}
-
-template <int NT>
-static hipError_t launch_nt(const GemvProblem& p, hipStream_t stream) {
-  switch (p.type) {
-    case kQ4_K: return launch_packed<kQ4_K, NT, 2>(p, stream);
-    case kQ6_K: return launch_packed<kQ6_K, NT, 2>(p, stream);
-    case kQ5_0: return launch_packed<kQ5_0, NT, 2>(p, stream);
-    case kQ8_0: return launch_packed<kQ8_0, NT, 2>(p, stream);
-    case kF32: return launch_f32<NT>(p, stream);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 template <int TYPE, int R>
@@ -403,6 +391,7 @@ static bool rows_path(const GemvProblem& p) {
 
 hipError_t gemv_launch(const GemvProblem& p, hipStream_t stream) {
   if (LLHIP_GEMV_MFMA && gemv_mfma_supported(p)) return gemv_mfma_launch(p, stream);
+  if (p.type != kF32 && p.tokens > 1) return gemm_launch(p, stream);
   if (rows_path(p)) {
     switch (p.type) {
       case kQ4_K: return launch_rows<kQ4_K, LLHIP_ROWS_Q4K>(p, stream);
@@ -412,11 +401,17 @@ hipError_t gemv_launch(const GemvProblem& p, hipStream_t stream) {
       default: break;
     }
   }
-  // Tokens are processed up to NT at a time (each chunk re-reads the
+  switch (p.type) {
+    case kQ4_K: return launch_packed<kQ4_K>(p, stream);
+    case kQ6_K: return launch_packed<kQ6_K>(p, stream);
+    case kQ5_0: return launch_packed<kQ5_0>(p, stream);
+    case kQ8_0: return launch_packed<kQ8_0>(p, stream);
+    case kF32: break;
+    default: return hipErrorInvalidValue;
+  }
+  // F32 tokens are processed up to NT at a time (each chunk re-reads the
   // weights); NT is capped so the staged activations fit in LDS.
-  const size_t per_token = p.type == kF32 ? (size_t)p.columns * sizeof(float)
-                                          : (size_t)(p.columns + (p.columns >> 4)) * sizeof(float);
-  const int fit = (int)std::min<size_t>(4, kMaxLdsBytes / per_token);
+  const int fit = (int)std::min<size_t>(4, kMaxLdsBytes / ((size_t)p.columns * sizeof(float)));
   if (fit < 1) return hipErrorInvalidValue;
   const int chunk = fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
   GemvProblem q = p;
@@ -425,9 +420,9 @@ hipError_t gemv_launch(const GemvProblem& p, hipStream_t stream) {
     q.x = p.x + (int64_t)t0 * p.x_stride;
     q.y = p.y + (int64_t)t0 * p.y_stride;
     hipError_t e;
-    if (q.tokens == 1) e = launch_nt<1>(q, stream);
-    else if (q.tokens == 2) e = launch_nt<2>(q, stream);
-    else e = launch_nt<4>(q, stream);
+    if (q.tokens == 1) e = launch_f32<1>(q, stream);
+    else if (q.tokens == 2) e = launch_f32<2>(q, stream);
+    else e = launch_f32<4>(q, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

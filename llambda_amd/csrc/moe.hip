@@ -330,7 +330,7 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
     // the experts' input ffn_latent_down * x (llambda.lisp:5883-5887) and
     // its split rows; the router and the shared expert keep x's
     GemvProblem g{p.lat_down_type, p.lat_down, row_bytes_of(p.lat_down_type, H), Li, H, x, H,
-                  tokens, p.lat, Li};
+                  tokens, p.lat, Li, true};
     e = gemv_launch(g, s);
     if (e != hipSuccess) return e;
     e = split_rows_launch(p.lat, tokens, Li, Li, p.lq, 2 * (int64_t)Li, p.lsum, Li / 16, s);
@@ -503,7 +503,7 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
              Lo, 0, static_cast<int*>(nullptr));
   if (e != hipSuccess) return e;
   GemvProblem g{p.lat_up_type, p.lat_up, row_bytes_of(p.lat_up_type, Lo), H, Lo, p.lat, Lo, tokens,
-                p.lat_y, H};
+                p.lat_y, H, true};
   e = gemv_launch(g, s);
   if (e != hipSuccess) return e;
   return launch(moe_latent_finish_kernel, dim3((H + 255) / 256, tokens), dim3(256), 0, s, p, y,

@@ -1,0 +1,170 @@
+"""Multi-token projections (gemm.hip) against 64-bit products of the oracle's
+dequantised weights.
+
+Bounds.  Every output's error is at most 2^-20 of its sum of |terms|: the
+activations carry 2^-23 relative error, and the longest run of fp32 adds into
+one sum is 8 chunks x (about 40 roundings in a chunk) with partial sums below
+the sum of |terms|, whose roundings add up at random (sqrt(320) 2^-24 < 2^-19,
+and the partial sums average half of the bound).  A Q4_K term counts as the
+three products it is formed from: sc (q - 8) d, 8 sc d and m dmin.  The 2-norm
+error of N(0, 1) activations stays below 3e-7 (an fp32 evaluation: 1.2e-7 to
+2.4e-7).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from llambda_amd import ggml, synthetic
+from llambda_amd.hip_backend import make_hip_session_packed
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [ggml.Q4_K, ggml.Q6_K, ggml.Q5_0, ggml.Q8_0]
+
+
+def _weights(type_tag, w, rows, columns):
+    return oracle.dequantize(type_tag, w, rows * columns).reshape(rows, columns).astype(np.float64)
+
+
+def _terms(type_tag, w, wd, rows, columns):
+    """|weight| per element as the kernel forms it."""
+    if type_tag != ggml.Q4_K:
+        return np.abs(wd)
+    b = w.reshape(-1, 144)
+    d = b[:, 0:2].copy().view(np.float16).astype(np.float64)
+    m = b[:, 2:4].copy().view(np.float16).astype(np.float64)
+    return np.abs(wd) + np.repeat(np.abs(d) * 63 * 16 + np.abs(m) * 63, 256, axis=1).reshape(rows, columns)
+
+
+def _run(s, x):
+    y = np.empty((x.shape[0], s.output_element_count), dtype=np.float32)
+    return s.run_batch_into(y, x, x.shape[0])
+
+
+def _check(type_tag, w, rows, columns, x, y, label, norm=True):
+    wd = _weights(type_tag, w, rows, columns)
+    ref = x.astype(np.float64) @ wd.T
+    bound = 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ _terms(type_tag, w, wd, rows, columns).T)
+    err = np.abs(y - ref)
+    assert np.all(err <= bound), (label, float((err / bound).max()))
+    if norm:
+        rel = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+        assert rel < 3e-7, (label, rel)
+
+
+# rows, columns (K-quants; block types), tokens: one row and one chunk, ragged
+# rows and tokens on both sides of every tile (16 x 16 to 256 x 64), one to
+# several chunks per wave group, more than eight chunks in one run of totals,
+# a last chunk of one 32-block, and grids that each tile shape serves
+SHAPES = [
+    (1, 256, 32, 2), (17, 512, 288, 3), (515, 2048, 1056, 16), (515, 2304, 1856, 17),
+    (1024, 2560, 2688, 33), (4096, 256, 544, 31), (4000, 768, 480, 65), (14000, 512, 96, 7),
+    (14000, 512, 320, 63), (14000, 256, 256, 130), (14300, 256, 224, 200), (1000, 5120, 4640, 300),
+]
+
+
+@pytest.mark.parametrize("type_tag", TYPES)
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_matches_64_bit_products(hip, type_tag, shape):
+    rows, wide, narrow, tokens = shape
+    columns = wide if type_tag in (ggml.Q4_K, ggml.Q6_K) else narrow
+    rng = np.random.default_rng(rows + tokens)
+    w = synthetic.packed(type_tag, rng, rows, columns)
+    x = synthetic.activations(rng, tokens, columns)
+    s = make_hip_session_packed(w, type_tag, rows, columns)
+    try:
+        y = _run(s, x)
+    finally:
+        s.close()
+    _check(type_tag, w, rows, columns, x, y, f"{ggml.NAMES[type_tag]} {shape}")
+
+
+@pytest.mark.parametrize("type_tag", TYPES)
+def test_extreme_activations_and_scales(hip, type_tag):
+    """Tokens of every magnitude beside each other, each exact to its own; an
+    infinity or a NaN stays in its token, and finite outputs that an infinity
+    reaches with a nonzero weight are infinite or NaN, never finite."""
+    rows, columns = 160, 1280
+    rng = np.random.default_rng(5)
+    w = synthetic.packed(type_tag, rng, rows, columns)
+    bb = ggml.block_bytes(type_tag)
+    blocks = w.reshape(-1, bb)
+    at = 208 if type_tag == ggml.Q6_K else 0
+    scales = np.array([2000.0, 256.0, -300.0, 6e-8, 0.0, 1e-5], dtype=np.float16)
+    blocks[:, at:at + 2] = rng.choice(scales, size=blocks.shape[0]).view(np.uint8).reshape(-1, 2)
+    x = synthetic.activations(rng, 23, columns)
+    for t, f in enumerate((1e-33, 1e-30, 1e28, 1e-20, 1e20, 0.0)):
+        x[t] = (x[t] * np.float32(f)).astype(np.float32)
+    x[7, ::3] *= np.float32(2.0 ** -12)
+    x[8, 5], x[9, 300], x[10, 700] = np.inf, -np.inf, np.nan
+    s = make_hip_session_packed(w, type_tag, rows, columns)
+    try:
+        with np.errstate(all="ignore"):
+            for first in (0, 3):  # both sides of the 16-token tiles
+                y = _run(s, np.ascontiguousarray(x[first:]))
+                fine = [t for t in range(first, 23) if t not in (8, 9, 10)]
+                _check(type_tag, w, rows, columns, x[fine], y[[t - first for t in fine]],
+                       f"extremes {ggml.NAMES[type_tag]}", norm=False)
+                wd = _weights(type_tag, w, rows, columns)
+                for t, k in ((8, 5), (9, 300), (10, 700)):
+                    reached = wd[:, k] != 0 if t < 10 else slice(None)
+                    assert not np.isfinite(y[t - first][reached]).any(), t
+                for t, k in ((8, 5), (9, 300)):
+                    if type_tag == ggml.Q4_K:  # its offset products may meet as inf - inf
+                        continue
+                    alone = (wd[:, k] != 0) & ~np.isnan(y[t - first])
+                    assert np.array_equal(np.sign(y[t - first][alone]), np.sign(x[t, k] * wd[alone, k]))
+    finally:
+        s.close()
+
+
+def test_device_rows_on_any_float(hip):
+    """x and y need float alignment only; neighbours of y stay untouched."""
+    import torch
+    rows, columns, tokens = 300, 768, 21
+    rng = np.random.default_rng(6)
+    for type_tag in TYPES:
+        w = synthetic.packed(type_tag, rng, rows, columns)
+        x = synthetic.activations(rng, tokens, columns)
+        s = make_hip_session_packed(w, type_tag, rows, columns)
+        try:
+            xd = torch.zeros(x.size + 3, device="cuda")
+            xd[1:1 + x.size] = torch.from_numpy(x.reshape(-1)).cuda()
+            yd = torch.full((tokens * rows + 6,), 7.0, device="cuda")
+            torch.cuda.synchronize()
+            s.run_device(xd[1:].data_ptr(), yd[3:].data_ptr(), tokens)
+            torch.cuda.synchronize()
+            y = yd.cpu().numpy()
+            assert np.all(y[:3] == 7.0) and np.all(y[-3:] == 7.0)
+            _check(type_tag, w, rows, columns, x, y[3:-3].reshape(tokens, rows), "offset rows")
+        finally:
+            s.close()
+
+
+def test_replays_in_a_graph(hip):
+    """A captured call replays with new activations, eager calls in between
+    (no memory is allocated by the call)."""
+    import torch
+    rows, columns, tokens = 515, 1024, 40
+    rng = np.random.default_rng(8)
+    w = synthetic.packed(ggml.Q4_K, rng, rows, columns)
+    s = make_hip_session_packed(w, ggml.Q4_K, rows, columns)
+    try:
+        xd = torch.zeros((tokens, columns), device="cuda")
+        yd = torch.zeros((tokens, rows), device="cuda")
+        ye = torch.zeros((tokens, rows), device="cuda")
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            s.run_device(xd.data_ptr(), yd.data_ptr(), tokens,
+                         torch.cuda.current_stream().cuda_stream)
+        for _ in range(3):
+            xd.copy_(torch.from_numpy(synthetic.activations(rng, tokens, columns)))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            s.run_device(xd.data_ptr(), ye.data_ptr(), tokens)
+            torch.cuda.synchronize()
+            assert torch.equal(yd, ye)
+    finally:
+        s.close()
