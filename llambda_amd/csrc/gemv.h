@@ -76,7 +76,7 @@ hipError_t gemv_fused_pair_launch(const GemvProblem& pa, const GemvFuse& fa, con
 bool gemv_mfma_supported(const GemvProblem& p);
 hipError_t gemv_mfma_launch(const GemvProblem& p, hipStream_t stream);
 
-// Q4_K / Q6_K / Q5_0 / Q8_0 products of two or more tokens on MFMA (gemm.hip).
+// Products of two or more tokens on MFMA, all types (gemm.hip).
 hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream);
 
 // Compute units of the current device (cached after the first call).

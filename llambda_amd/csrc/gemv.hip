@@ -4,8 +4,8 @@
 // Q5_0, Q8_0 (units.h) and F32, i.e. %gguf-model-matrix-vector-multiply-into
 // (llambda.lisp:4542-4658) on one MI355X.
 //
-// Several tokens of packed rows run on MFMA (gemm.hip), one token of Q4_K and
-// Q6_K too (gemv_mfma.hip); here are one token of the other rows, and F32.
+// Several tokens run on MFMA (gemm.hip), one token of Q4_K and Q6_K too
+// (gemv_mfma.hip); here is one token of the other types.
 // Launch shape of rows whose K 64 does not divide: 256-thread workgroups (4
 // wavefronts).  Each workgroup copies the token's activations into LDS once,
 // with the sums of every 16-element group, then its wavefronts stream rows: a
@@ -161,43 +161,31 @@ gemv_rows_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int
   }
 }
 
-// F32 rows (the router): one float4 of W per lane per step.
-template <int NT>
+// F32 rows (the router), one token: one float4 of W per lane per step.
 __global__ void __launch_bounds__(256)
 gemv_f32_kernel(const float* __restrict__ w, int rows, int K, const float* __restrict__ x,
-                int64_t x_stride, int ntok, float* __restrict__ y, int64_t y_stride) {
+                float* __restrict__ y) {
   extern __shared__ float smem[];
   float* xs = smem;
-  for (int i = threadIdx.x; i < NT * K; i += blockDim.x) {
-    const int tok = i / K, k = i - tok * K;
-    xs[i] = tok < ntok ? x[tok * x_stride + k] : 0.f;
-  }
+  for (int i = threadIdx.x; i < K; i += blockDim.x) xs[i] = x[i];
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int waves_per_block = blockDim.x >> 6;
   const int n4 = K >> 2;
   for (int row = blockIdx.x * waves_per_block + wave; row < rows; row += gridDim.x * waves_per_block) {
-    float acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = 0.f;
+    float acc = 0.f;
     const float4* wr = reinterpret_cast<const float4*>(w + (int64_t)row * K);
     for (int k4 = lane; k4 < n4; k4 += kWave) {
       const float4 a = wr[k4];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float4 b = reinterpret_cast<const float4*>(xs + t * K)[k4];
-        acc[t] = fmaf(a.x, b.x, acc[t]);
-        acc[t] = fmaf(a.y, b.y, acc[t]);
-        acc[t] = fmaf(a.z, b.z, acc[t]);
-        acc[t] = fmaf(a.w, b.w, acc[t]);
-      }
+      const float4 b = reinterpret_cast<const float4*>(xs)[k4];
+      acc = fmaf(a.x, b.x, acc);
+      acc = fmaf(a.y, b.y, acc);
+      acc = fmaf(a.z, b.z, acc);
+      acc = fmaf(a.w, b.w, acc);
     }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const float v = segment_sum<kWave>(acc[t]);
-      if (lane == 0 && t < ntok) y[t * y_stride + row] = v;
-    }
+    const float v = segment_sum<kWave>(acc);
+    if (lane == 0) y[row] = v;
   }
 }
 
@@ -345,14 +333,14 @@ static hipError_t launch_packed(const GemvProblem& p, hipStream_t stream) {
                          (int)p.rows, (int)p.columns, p.x, p.y, lpr_log2);
 }
 
-template <int NT>
 static hipError_t launch_f32(const GemvProblem& p, hipStream_t stream) {
   const int needed = (int)((p.rows + 3) / 4);
-  const size_t lds = (size_t)NT * p.columns * sizeof(float);
+  const size_t lds = (size_t)p.columns * sizeof(float);
+  if (lds > kMaxLdsBytes) return hipErrorInvalidValue;
   const int grid = std::max(1, std::min(needed, device_cu_count() * 8));
-  return launch_with_lds(gemv_f32_kernel<NT>, grid, lds, stream,
+  return launch_with_lds(gemv_f32_kernel, grid, lds, stream,
                          reinterpret_cast<const float*>(p.weights), (int)p.rows, (int)p.columns,
-                         p.x, p.x_stride, p.tokens, p.y, p.y_stride);
+                         p.x, p.y);
 }
 
 template <int TYPE, int R>
@@ -391,7 +379,7 @@ static bool rows_path(const GemvProblem& p) {
 
 hipError_t gemv_launch(const GemvProblem& p, hipStream_t stream) {
   if (LLHIP_GEMV_MFMA && gemv_mfma_supported(p)) return gemv_mfma_launch(p, stream);
-  if (p.type != kF32 && p.tokens > 1) return gemm_launch(p, stream);
+  if (p.tokens > 1) return gemm_launch(p, stream);
   if (rows_path(p)) {
     switch (p.type) {
       case kQ4_K: return launch_rows<kQ4_K, LLHIP_ROWS_Q4K>(p, stream);
@@ -406,26 +394,9 @@ hipError_t gemv_launch(const GemvProblem& p, hipStream_t stream) {
     case kQ6_K: return launch_packed<kQ6_K>(p, stream);
     case kQ5_0: return launch_packed<kQ5_0>(p, stream);
     case kQ8_0: return launch_packed<kQ8_0>(p, stream);
-    case kF32: break;
+    case kF32: return launch_f32(p, stream);
     default: return hipErrorInvalidValue;
   }
-  // F32 tokens are processed up to NT at a time (each chunk re-reads the
-  // weights); NT is capped so the staged activations fit in LDS.
-  const int fit = (int)std::min<size_t>(4, kMaxLdsBytes / ((size_t)p.columns * sizeof(float)));
-  if (fit < 1) return hipErrorInvalidValue;
-  const int chunk = fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
-  GemvProblem q = p;
-  for (int t0 = 0; t0 < p.tokens; t0 += chunk) {
-    q.tokens = std::min(chunk, p.tokens - t0);
-    q.x = p.x + (int64_t)t0 * p.x_stride;
-    q.y = p.y + (int64_t)t0 * p.y_stride;
-    hipError_t e;
-    if (q.tokens == 1) e = launch_f32<1>(q, stream);
-    else if (q.tokens == 2) e = launch_f32<2>(q, stream);
-    else e = launch_f32<4>(q, stream);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
 }
 
 hipError_t dequant_launch(int type, const uint8_t* w, int64_t row_bytes, int64_t rows,

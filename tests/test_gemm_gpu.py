@@ -23,6 +23,8 @@ TYPES = [ggml.Q4_K, ggml.Q6_K, ggml.Q5_0, ggml.Q8_0]
 
 
 def _weights(type_tag, w, rows, columns):
+    if type_tag == ggml.F32:
+        return w.view(np.float32).reshape(rows, columns).astype(np.float64)
     return oracle.dequantize(type_tag, w, rows * columns).reshape(rows, columns).astype(np.float64)
 
 
@@ -118,12 +120,31 @@ def test_extreme_activations_and_scales(hip, type_tag):
         s.close()
 
 
+@pytest.mark.parametrize("shape", [(1, 4, 2), (33, 260, 16), (515, 1028, 17), (512, 2048, 33),
+                                   (96, 4100, 130)], ids=lambda s: "x".join(map(str, s)))
+def test_f32_rows(hip, shape):
+    rows, columns, tokens = shape
+    rng = np.random.default_rng(rows)
+    w = synthetic.packed(ggml.F32, rng, rows, columns)
+    x = synthetic.activations(rng, tokens, columns)
+    s = make_hip_session_packed(w, ggml.F32, rows, columns)
+    try:
+        y = _run(s, x)
+        again = _run(s, np.ascontiguousarray(x[:2]))  # one order of sums in every batch
+    finally:
+        s.close()
+    wd = w.view(np.float32).reshape(rows, columns).astype(np.float64)
+    bound = 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(wd).T)
+    assert np.all(np.abs(y - x.astype(np.float64) @ wd.T) <= bound)
+    assert np.array_equal(again, y[:2])
+
+
 def test_device_rows_on_any_float(hip):
     """x and y need float alignment only; neighbours of y stay untouched."""
     import torch
     rows, columns, tokens = 300, 768, 21
     rng = np.random.default_rng(6)
-    for type_tag in TYPES:
+    for type_tag in TYPES + [ggml.F32]:
         w = synthetic.packed(type_tag, rng, rows, columns)
         x = synthetic.activations(rng, tokens, columns)
         s = make_hip_session_packed(w, type_tag, rows, columns)
