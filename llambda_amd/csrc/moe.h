@@ -148,11 +148,13 @@ struct MoeGemmArgs {
 };
 
 // Router logits of T tokens (fp32 MFMA) as router_slices(H) partial sums
-// part[slice][t][e] (row stride ld), and the split rows of x (q, s).
+// part[slice][t][e] (row stride ld), and the split rows of x (q, s), or with
+// `image` (kQ4_K, kQ6_K; H of whole 256-element chunks) its f16 operand images
+// for products with that type.
 int router_slices(int H);
 hipError_t router_mfma_launch(const float* x, int T, const float* R, int Er, int H, float* part,
                               int ld, uint16_t* q, int64_t q_stride, float* s, int64_t s_stride,
-                              hipStream_t stream);
+                              int image, hipStream_t stream);
 // The split rows (format above router_mfma_launch's q, s) of T rows of K
 // fp32 elements, K % 32 == 0, rows x_stride floats apart.
 hipError_t split_rows_launch(const float* x, int T, int K, int64_t x_stride, uint16_t* q,
@@ -183,6 +185,16 @@ bool moe_tiled_type(int type);
 int64_t moe_slab_bytes(int type, int64_t rows, int64_t columns);
 hipError_t moe_tile_launch(int type, const uint8_t* src, int64_t slabs, int64_t rows,
                            int64_t columns, uint8_t* dst, hipStream_t stream);
+
+// K-quant swiglu layers of whole 256-element chunks, two or more tokens
+// (moe_f16.hip): x as f16 operand images (from the router launch), gate|up
+// with the activation (fp32 rows in the split activations' buffer), down.  token_tiles: 1 or 2 tiles of 16 pairs per chunk
+// of the table (each output's bits are the same).
+bool moe_f16_supported(const MoePlan& p);
+hipError_t moe_f16_up_launch(int type, const MoeGemmArgs& a, int token_tiles, int max_chunks,
+                             hipStream_t stream);
+hipError_t moe_f16_down_launch(int type, const MoeGemmArgs& a, int token_tiles, int max_chunks,
+                               hipStream_t stream);
 
 // One token's down products and their combine in one launch (moe_mfma.hip):
 // a.chunks / a.chunk_counts / a.perm as topk_gate_kernel writes them for a

@@ -323,8 +323,9 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
   const int act_w = std::max(p.ffn, p.shared_ffn);
   const int64_t xs_stride = H / 16, as_stride = act_w / 16;
   const int er = E + ((p.variant == kQwen3Next && has_shared) ? 1 : 0);
+  const bool f16 = tokens > 1 && moe_f16_supported(p);
   hipError_t e = router_mfma_launch(x, tokens, p.router, er, H, p.router_part, E + 1, p.xq,
-                                    2 * (int64_t)H, p.xsum, xs_stride, s);
+                                    2 * (int64_t)H, p.xsum, xs_stride, f16 ? p.up_type : 0, s);
   if (e != hipSuccess) return e;
   if (Li) {
     // the experts' input ffn_latent_down * x (llambda.lisp:5883-5887) and
@@ -417,6 +418,9 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
     a.expert_stride = p.up_g_stride;
     a.s_w0 = p.sh_up_g;
   }
+  if (f16)
+    e = moe_f16_up_launch(p.up_type, a, mt, routed_chunks + (joint_up ? shared_chunks : 0), s);
+  else
   e = moe_gemm_launch(p.up_type, epi, a, mt,
                       fuse_gate ? K + (joint_up ? 1 : 0)
                                 : routed_chunks + (joint_up ? shared_chunks : 0),
@@ -480,7 +484,9 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
     a.expert_stride = p.down_g_stride;
     a.s_w0 = p.sh_down_g;
   }
-  e = moe_gemm_launch(p.down_type, kEpiDown, a, mt, routed_chunks + (joint_down ? shared_chunks : 0), s);
+  const int down_chunks = routed_chunks + (joint_down ? shared_chunks : 0);
+  e = f16 ? moe_f16_down_launch(p.down_type, a, mt, down_chunks, s)
+          : moe_gemm_launch(p.down_type, kEpiDown, a, mt, down_chunks, s);
   if (e != hipSuccess) return e;
   if (has_shared && !joint_down) {
     a = down;

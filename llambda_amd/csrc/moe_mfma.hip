@@ -64,6 +64,7 @@
 #include "activations.h"
 #include "mfma.h"
 #include "moe.h"
+#include "moe_f16.h"
 #include "moe_gate.h"
 
 #include <algorithm>
@@ -146,7 +147,9 @@ constexpr int kRouterSlice = 512;
 // once per GE expert tiles instead of once per tile); wave w < GE adds the
 // eight wave sums of expert tile w.  Every tile's arithmetic is the same for
 // any GE.
-template <int GE>
+// IMAGE: 0, or the K-quant type whose products read the tokens as f16 images
+// (moe_f16.h) instead of split rows.
+template <int GE, int IMAGE>
 __global__ void __launch_bounds__(64 * kRouterWaves)
 router_mfma_kernel(const float* __restrict__ x, int T, const float* __restrict__ R, int Er, int H,
                    float* __restrict__ part, int ld, uint16_t* __restrict__ q, int64_t q_stride,
@@ -175,12 +178,35 @@ router_mfma_kernel(const float* __restrict__ x, int T, const float* __restrict__
   }
   load_r(eg, rb);
   if (blockIdx.x == 0) {
-    const int octets = min(kRouterSlice, H - k0) >> 3, ofirst = k0 >> 3;
-    for (int idx = threadIdx.x; idx < 16 * octets; idx += 64 * kRouterWaves) {
-      const int tt = idx / octets, o = ofirst + idx - tt * octets;
-      if (t0 + tt < T)
-        split_octet(x + (int64_t)(t0 + tt) * H, o, q + (int64_t)(t0 + tt) * q_stride,
-                    s + (int64_t)(t0 + tt) * s_stride);
+    if constexpr (IMAGE != 0) {
+      // a wavefront per (token, chunk) of the slice
+      using W = ExpertW<IMAGE>;
+      const int chunks = min(kRouterSlice, H - k0) >> 8;
+      for (int idx = wave; idx < 16 * chunks; idx += kRouterWaves) {
+        const int c = idx >> 4, t = t0 + (idx & 15);
+        if (t >= T) continue;
+        const floatx4 v =
+            *reinterpret_cast<const floatx4*>(x + (int64_t)t * H + k0 + 256 * c + 4 * lane);
+        uint2 hi, lo;
+        u32x4 side;
+        split_chunk<W>(v, lane, hi, lo, side);
+        int g, st, high;
+        W::place(lane, g, st, high);
+        uint8_t* row = reinterpret_cast<uint8_t*>(q + t * q_stride) + 1024 * ((k0 >> 8) + c);
+        uint2* at = reinterpret_cast<uint2*>(row + 64 * st + 16 * g + 8 * high);
+        at[0] = hi;
+        at[64] = lo;
+        if ((lane & 15) == 0)
+          (reinterpret_cast<u32x4*>(s + t * s_stride) + 4 * ((k0 >> 8) + c))[lane >> 4] = side;
+      }
+    } else {
+      const int octets = min(kRouterSlice, H - k0) >> 3, ofirst = k0 >> 3;
+      for (int idx = threadIdx.x; idx < 16 * octets; idx += 64 * kRouterWaves) {
+        const int tt = idx / octets, o = ofirst + idx - tt * octets;
+        if (t0 + tt < T)
+          split_octet(x + (int64_t)(t0 + tt) * H, o, q + (int64_t)(t0 + tt) * q_stride,
+                      s + (int64_t)(t0 + tt) * s_stride);
+      }
     }
   }
 #pragma unroll
@@ -223,9 +249,10 @@ router_mfma_kernel(const float* __restrict__ x, int T, const float* __restrict__
 
 int router_slices(int H) { return (H + kRouterSlice - 1) / kRouterSlice; }
 
-hipError_t router_mfma_launch(const float* x, int T, const float* R, int Er, int H, float* part,
-                              int ld, uint16_t* q, int64_t q_stride, float* s, int64_t s_stride,
-                              hipStream_t stream) {
+template <int IMAGE>
+static hipError_t launch_router(const float* x, int T, const float* R, int Er, int H, float* part,
+                                int ld, uint16_t* q, int64_t q_stride, float* s, int64_t s_stride,
+                                hipStream_t stream) {
   // batches of 32 token tiles or more take eight expert tiles per
   // workgroup, of 16 or more four (a grid of 576 workgroups for 256 tokens
   // and 513 rows: Qwen3Next B=256 0.408 -> 0.404 ms against eight), smaller
@@ -233,18 +260,29 @@ hipError_t router_mfma_launch(const float* x, int T, const float* R, int Er, int
   const int etiles = (Er + 15) / 16, ttiles = (T + 15) / 16;
   if (ttiles >= 32) {
     const dim3 grid((etiles + 7) / 8, ttiles, router_slices(H));
-    hipLaunchKernelGGL(router_mfma_kernel<8>, grid, dim3(64 * kRouterWaves), 0, stream, x, T, R, Er,
-                       H, part, ld, q, q_stride, s, s_stride);
+    hipLaunchKernelGGL((router_mfma_kernel<8, IMAGE>), grid, dim3(64 * kRouterWaves), 0, stream, x,
+                       T, R, Er, H, part, ld, q, q_stride, s, s_stride);
   } else if (ttiles >= 16) {
     const dim3 grid((etiles + 3) / 4, ttiles, router_slices(H));
-    hipLaunchKernelGGL(router_mfma_kernel<4>, grid, dim3(64 * kRouterWaves), 0, stream, x, T, R, Er,
-                       H, part, ld, q, q_stride, s, s_stride);
+    hipLaunchKernelGGL((router_mfma_kernel<4, IMAGE>), grid, dim3(64 * kRouterWaves), 0, stream, x,
+                       T, R, Er, H, part, ld, q, q_stride, s, s_stride);
   } else {
     const dim3 grid(etiles, ttiles, router_slices(H));
-    hipLaunchKernelGGL(router_mfma_kernel<1>, grid, dim3(64 * kRouterWaves), 0, stream, x, T, R, Er,
-                       H, part, ld, q, q_stride, s, s_stride);
+    hipLaunchKernelGGL((router_mfma_kernel<1, IMAGE>), grid, dim3(64 * kRouterWaves), 0, stream, x,
+                       T, R, Er, H, part, ld, q, q_stride, s, s_stride);
   }
   return hipGetLastError();
+}
+
+hipError_t router_mfma_launch(const float* x, int T, const float* R, int Er, int H, float* part,
+                              int ld, uint16_t* q, int64_t q_stride, float* s, int64_t s_stride,
+                              int image, hipStream_t stream) {
+  switch (image) {
+    case 0: return launch_router<0>(x, T, R, Er, H, part, ld, q, q_stride, s, s_stride, stream);
+    case kQ4_K: return launch_router<kQ4_K>(x, T, R, Er, H, part, ld, q, q_stride, s, s_stride, stream);
+    case kQ6_K: return launch_router<kQ6_K>(x, T, R, Er, H, part, ld, q, q_stride, s, s_stride, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 // ------------------------------------------------------ B operand per type
