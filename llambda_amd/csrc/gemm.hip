@@ -691,11 +691,12 @@ gemm_many_kernel(GemmArgs a) {
 // Tiles of 32 rows x 16 JT tokens on v_mfma_f32_16x16x4_f32; the workgroup's
 // eight waves deal the 16-element pieces of K among themselves (lane (n, g)
 // loads elements 4g .. 4g + 3 of a piece of row or token n: 64 contiguous
-// bytes a row), their sums added in wave order.  Each token's sums run in one
+// bytes a row).  Each token's sums run in one
 // order whatever the batch and JT.  Bound by the loads' latency at few tokens
-// (512 x 2048, 7 tokens: 19.8 -> 11.9 us), by the fp32 MFMA at many (2048 x
-// 4096, 512 tokens: 3.6 ms in passes of four tokens on the VALU -> 0.128 ms,
-// 67 of 157 TFLOP/s); errors against 64 bits 1.1e-7 (1.2e-7 to 1.6e-7 before).
+// (512 x 2048, 7 tokens: 19.8 -> 11.7 us), by the fp32 MFMA at many (2048 x
+// 4096, 512 tokens: 3.6 ms in passes of four tokens on the VALU -> 0.123 ms,
+// 70 of 157 TFLOP/s); errors against 64 bits 0.8e-7 to 1.0e-7 (0.8e-7 to
+// 1.6e-7 before).
 constexpr int kF32Waves = 8;
 template <int JT>
 __global__ void __launch_bounds__(64 * kF32Waves)
@@ -731,18 +732,21 @@ gemm_f32_kernel(GemmArgs a) {
       for (int j = 0; j < JT; ++j)
         x[p][j] = in ? (floatx4)*reinterpret_cast<const floatx4a4*>(xr[j] + k) : floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    // each piece's four products in a sum of their own, added pairwise
+    // every product in a sum of its own (four elements), added pairwise: a
+    // piece's four products in one running sum were 20% further off 64 bits
+    // than the VALU's sums had been at K = 424
     floatx4 sum[PIECES][RT][JT];
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int p = 0; p < PIECES; ++p)
 #pragma unroll
-      for (int p = 0; p < PIECES; ++p)
+      for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-          for (int j = 0; j < JT; ++j)
-            sum[p][r][j] = mfma4f32(x[p][j][e], w[p][r][e],
-                                    e ? sum[p][r][j] : floatx4{0.f, 0.f, 0.f, 0.f});
+        for (int j = 0; j < JT; ++j) {
+          const floatx4 &u = x[p][j], &v = w[p][r];
+          sum[p][r][j] = (mfma4f32(u[0], v[0], zero) + mfma4f32(u[1], v[1], zero)) +
+                         (mfma4f32(u[2], v[2], zero) + mfma4f32(u[3], v[3], zero));
+        }
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -758,8 +762,9 @@ gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < RT * JT; ++i) {
     floatx4& t = tot[i / JT][i % JT];
-#pragma unroll
-    for (int q = 0; q < kF32Waves - 1; ++q) t += red[q][i][lane];
+    static_assert(kF32Waves == 8, "the sum below");
+    t = ((t + red[0][i][lane]) + (red[1][i][lane] + red[2][i][lane])) +
+        ((red[3][i][lane] + red[4][i][lane]) + (red[5][i][lane] + red[6][i][lane]));
     const int row = row0 + 16 * (i / JT) + n;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -769,8 +774,68 @@ gemm_f32_kernel(GemmArgs a) {
   }
 }
 
+// F32 rows of two to four tokens: a workgroup takes 8 / NT rows and its
+// waves take turns at the columns, a float4 of each row and token per lane
+// and turn, straight from memory.  Bound by latency up to some thousand rows:
+// a wave's loads of one turn are all in flight together, and nothing is
+// staged.  Against rows read from LDS-staged tokens by one wave each, and
+// against the MFMA tiles below five tokens: 512 x 2048, 2 tokens 6.5 and 10.8
+// -> 3.9 us; 1024 x 4096, 4 tokens 28.0 and 20.4 -> 6.2 us; 20000 x 2048, 2
+// tokens 36.5 and 46.0 -> 28.6 us (5.7 TB/s).  From five tokens on the tiles
+// win: 512 x 2048, 5 tokens 15.0 -> 11.2 us.
+constexpr int kFewWaves = 4, kFewSums = 8;
+template <int NT>
+__global__ void __launch_bounds__(64 * kFewWaves)
+gemm_f32_few_kernel(GemmArgs a) {
+  constexpr int R = kFewSums / NT;
+  __shared__ float red[kFewWaves][kFewSums];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row0 = blockIdx.x * R;
+  const float* wr[R];
+  const float* xr[NT];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    wr[r] = reinterpret_cast<const float*>(a.w) + (int64_t)min(row0 + r, a.rows - 1) * a.K;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) xr[t] = a.x + (int64_t)min(t, a.tokens - 1) * a.x_stride;
+  float acc[R][NT] = {};
+#pragma unroll 2
+  for (int k = 4 * (64 * wave + lane); k < a.K; k += 4 * 64 * kFewWaves) {  // K is a multiple of 4
+    floatx4 w[R], x[NT];
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = *reinterpret_cast<const floatx4a4*>(wr[r] + k);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) x[t] = *reinterpret_cast<const floatx4a4*>(xr[t] + k);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[r][t] += fmaf(w[r][1], x[t][1], w[r][0] * x[t][0]) + fmaf(w[r][3], x[t][3], w[r][2] * x[t][2]);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float v = segment_sum<kWave>(acc[r][t]);
+      if (lane == 0) red[wave][r * NT + t] = v;
+    }
+  __syncthreads();
+  if (threadIdx.x >= kFewSums) return;
+  const int row = row0 + threadIdx.x / NT, t = threadIdx.x % NT;
+  if (row < a.rows && t < a.tokens)
+    a.y[(int64_t)t * a.y_stride + row] = (red[0][threadIdx.x] + red[1][threadIdx.x]) +
+                                         (red[2][threadIdx.x] + red[3][threadIdx.x]);
+}
+
 // ------------------------------------------------------------------ host
-static hipError_t launch_f32(const GemmArgs& a, hipStream_t stream) {
+static hipError_t launch_f32(const GemmArgs& a, bool one_order, hipStream_t stream) {
+  if (a.tokens <= 4 && !one_order) {
+    const auto kernel = a.tokens <= 2 ? gemm_f32_few_kernel<2> : gemm_f32_few_kernel<4>;
+    const int rows = kFewSums / (a.tokens <= 2 ? 2 : 4);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.rows + rows - 1) / rows)),
+                       dim3(64 * kFewWaves), 0, stream, a);
+    return hipGetLastError();
+  }
   const unsigned rows = (unsigned)((a.rows + 31) / 32);
   // tokens in launches of at most 65535 tiles of 32
   GemmArgs q = a;
@@ -884,7 +949,7 @@ hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream) {
     case kQ6_K: return launch_type<kQ6_K>(a, p.one_order, stream);
     case kQ5_0: return launch_type<kQ5_0>(a, p.one_order, stream);
     case kQ8_0: return launch_type<kQ8_0>(a, p.one_order, stream);
-    case kF32: return launch_f32(a, stream);
+    case kF32: return launch_f32(a, p.one_order, stream);
     default: return hipErrorInvalidValue;
   }
 }
