@@ -11,6 +11,8 @@
 //     activation fused (silu(g)*u, or relu(u)^2)
 //   5 grouped down: down rows against the chunk's activations, per pair
 //   6 combine in rank order, then the shared expert
+// K-quant swiglu layers (moe_f16_supported) run 4 and 5 of two or more tokens
+// on f16 operand images (moe_f16.hip), which 1 forms from x.
 // A Nemotron-H layer with ffn_latent_down also runs that projection on x
 // and splits its output after 1 (the routed up products read it); with
 // ffn_latent_up, 6 forms the latent-wide weighted sum, then ffn_latent_up and

@@ -8,6 +8,8 @@
 //   moe_gemm_kernel     the grouped expert products over the chunk table
 //                       (expert, up to 16*MT (token, rank) pairs): gate/up
 //                       with silu(g)*u or relu(u)^2 fused, or down.
+//                       Layers that moe_f16_supported accepts take it at
+//                       one token only.
 //
 // Expert products.  The weights stay the tensor's GGUF super-blocks.  Each
 // wavefront owns 16-row subtiles of one or two matrices (gate and up side by
