@@ -107,26 +107,32 @@ struct GemmW<kQ6_K> {
   }
 };
 
-// Scales of a 32-block type: d of blocks 2g and 2g + 1, both / 256 where one
-// of the wave's is 256 or more (d q would leave f16's range).  Blocks past
-// the row's end (the last chunk of a K that 256 does not divide) count 0.
+// Scales of a 32-block type: d of blocks 2g and 2g + 1.  Blocks past the row's
+// end (the last chunk of a K that 256 does not divide) count 0.  A |d| of 256
+// or more would leave f16's range in d q: such blocks count 0 in a chunk's
+// products, and the wave adds them in a pass of their own, as d / 256 (d / 256
+// of the small d beside them would fall among f16's subnormals).
 struct BlockScale {
   half2v sl, sh;
-  float d;
+  uint64_t large;  // lanes with a |d| of 256 or more
   __device__ __forceinline__ void set(uint32_t d0, uint32_t d1, int g, int blocks) {
     d0 = 2 * g < blocks ? d0 & 0xFFFFu : 0u;
     d1 = 2 * g + 1 < blocks ? d1 & 0xFFFFu : 0u;
-    const bool wide = (d0 & 0x7FFFu) >= 0x5C00u || (d1 & 0x7FFFu) >= 0x5C00u;
+    large = __ballot(is_large(d0) || is_large(d1));
+    d0 = is_large(d0) ? 0u : d0;
+    d1 = is_large(d1) ? 0u : d1;
     sl = as_half2(d0 | (d0 << 16));
     sh = as_half2(d1 | (d1 << 16));
-    d = 1.f;
-    if (__any(wide)) {
-      const half2v f = splat2((_Float16)(1.f / 256.f));
-      sl = sl * f;
-      sh = sh * f;
-      d = 256.f;
-    }
   }
+  __device__ __forceinline__ void set_large(uint32_t d0, uint32_t d1, int g, int blocks) {
+    const half2v f = splat2((_Float16)(1.f / 256.f));
+    d0 = 2 * g < blocks && is_large(d0) ? d0 & 0xFFFFu : 0u;
+    d1 = 2 * g + 1 < blocks && is_large(d1) ? d1 & 0xFFFFu : 0u;
+    large = __ballot((d0 | d1) != 0u);
+    sl = as_half2(d0 | (d0 << 16)) * f;
+    sh = as_half2(d1 | (d1 << 16)) * f;
+  }
+  static __device__ __forceinline__ bool is_large(uint32_t d) { return (d & 0x7FFFu) >= 0x5C00u; }
 };
 
 template <>
@@ -141,8 +147,8 @@ struct GemmW<kQ8_0> : QuadsByGroup {
   struct Finish {
     float d;
   };
-  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale& c, int) {
-    f.d = c.d;
+  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale&, int) {
+    f.d = 1.f;
   }
   static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g,
                                               int blocks) {
@@ -153,6 +159,9 @@ struct GemmW<kQ8_0> : QuadsByGroup {
   }
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[8] >> 16, g, r.blocks);
+  }
+  static __device__ __forceinline__ void prepare_large(Scale& c, const Raw& r, int g) {
+    c.set_large(r.w[0], r.w[8] >> 16, g, r.blocks);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
                                               int s) {
@@ -182,8 +191,8 @@ struct GemmW<kQ5_0> : QuadsByGroup {
   struct Finish {
     float d;
   };
-  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale& c, int) {
-    f.d = c.d;
+  static __device__ __forceinline__ void finish(Finish& f, const Raw&, const Scale&, int) {
+    f.d = 1.f;
   }
   static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g,
                                               int blocks) {
@@ -194,6 +203,9 @@ struct GemmW<kQ5_0> : QuadsByGroup {
   }
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[5] >> 16, g, r.blocks);
+  }
+  static __device__ __forceinline__ void prepare_large(Scale& c, const Raw& r, int g) {
+    c.set_large(r.w[0], r.w[5] >> 16, g, r.blocks);
   }
   // element 4s + b: nibble s >> 2 of qs byte 4 (s & 3) + b, fifth bit 4s + b of qh
   static __device__ __forceinline__ uint32_t code(uint32_t qs, uint32_t qh, int s) {
@@ -232,6 +244,90 @@ struct GemmArgs {
   int row_tiles, token_tiles;  // gemm_many_kernel
 };
 
+// The large scales' products (BlockScale) of one row tile's chunk, JT token
+// tiles: operand(st, j, hi, lo) gives step st's activations of tile j.  Rows
+// without a large scale keep their totals (their products are 0 times x).
+template <typename W, int JT, typename Operand, typename Inverse>
+__device__ __forceinline__ void add_large(floatx4 (&tot)[JT], const typename W::Raw& raw,
+                                          int lane, Operand operand, Inverse inverse) {
+  // the codes anew: shared with the chunk's other products they would be kept
+  // in registers from here on
+  typename W::Raw own = raw;
+#pragma unroll
+  for (uint32_t& v : own.w) v = opaque(v);
+  typename W::Scale sc;
+  W::prepare_large(sc, own, lane >> 4);
+  floatx4 blk[JT];
+#pragma unroll
+  for (int j = 0; j < JT; ++j) blk[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    half8v bh, bl;
+    W::frag(bh, bl, own, sc, st);
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      half8v hi, lo;
+      operand(st, j, hi, lo);
+      blk[j] = mfma_f16(lo, bh, blk[j]);
+      blk[j] = mfma_f16(hi, bl, blk[j]);
+      blk[j] = mfma_f16(hi, bh, blk[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const uint64_t m = sc.large;
+  const uint32_t rows = (uint32_t)(m | (m >> 16) | (m >> 32) | (m >> 48));
+  if ((rows >> (lane & 15)) & 1u) {
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      const floatx4 inv = inverse(j);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tot[j][i] = fmaf(256.f * inv[i], blk[j][i], tot[j][i]);
+    }
+  }
+}
+
+// The activations of lane (token n, group g) in chunk c, xr the token's row:
+// split into ah and al, with 1 / s of the tokens of D's rows in inv.
+template <typename W>
+__device__ __forceinline__ void split_tokens(half8v (&ah)[8], half8v (&al)[8], floatx4& inv,
+                                             const float* xr, int c, int K, int g) {
+  floatx4 v[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int k = 256 * c + W::quad(g, q >> 1, q & 1);
+    v[q] = (!W::kBlocks32 || k < K) ? (floatx4)*reinterpret_cast<const floatx4a4*>(xr + k)
+                                    : floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  float top = 0.f;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) top = abs_max4(top, v[q]);
+  top = fmaxf(top, __shfl_xor(top, 16));
+  top = fmaxf(top, __shfl_xor(top, 32));
+  float s, inv1;
+  chunk_scale(top, s, inv1);
+  const bool special = __any(infinite(top));
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    uint2 h0, l0, h1, l1;
+    split_quad(v[2 * st], s, h0, l0);
+    split_quad(v[2 * st + 1], s, h1, l1);
+    ah[st] = __builtin_bit_cast(half8v, u32x4{h0.x, h0.y, h1.x, h1.y});
+    al[st] = __builtin_bit_cast(half8v, u32x4{l0.x, l0.y, l1.x, l1.y});
+  }
+  if (special) {
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      const u32x4 h = __builtin_bit_cast(u32x4, ah[st]);
+      u32x4 l = __builtin_bit_cast(u32x4, al[st]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) l[i] = drop_inf(h[i], l[i]);
+      al[st] = __builtin_bit_cast(half8v, l);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) inv[i] = __shfl(inv1, 4 * g + i);
+}
+
 // --------------------------------------------------------- few tokens
 // One token tile of 16 per workgroup column; the workgroup's KW waves share
 // 16 RT rows and deal the chunks among themselves, each wave holding its
@@ -257,6 +353,7 @@ gemm_few_kernel(GemmArgs a) {
   floatx4 tot[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+  uint64_t large = 0;
 
   for (int c = kw; c < a.chunks; c += KW) {
     const int blocks = W::kBlocks32 ? min(8, (a.K >> 5) - 8 * c) : 8;
@@ -322,6 +419,7 @@ gemm_few_kernel(GemmArgs a) {
     for (int r = 0; r < RT; ++r) {
       typename W::Scale sc;
       W::prepare(sc, raw[r], g);
+      if constexpr (W::kBlocks32) large |= sc.large;
       // the small products first: each add to the sums rounds in proportion
       // to what they have reached
       floatx4 blk = {0.f, 0.f, 0.f, 0.f};
@@ -337,6 +435,26 @@ gemm_few_kernel(GemmArgs a) {
       typename W::Finish fin;
       W::finish(fin, raw[r], sc, g);
       add_products<W>(tot[r], blk, inv, fin, sums);
+    }
+  }
+  if constexpr (W::kBlocks32) {
+    // the chunks again if any has a large scale (out of the loop above, whose
+    // one block of decode and products runs 2 to 5% longer with a branch in it)
+    if (large) [[unlikely]] {
+      for (int c = kw; c < a.chunks; c += KW) {
+        half8v ah[8], al[8];
+        floatx4 inv;
+        split_tokens<W>(ah, al, inv, xr, c, a.K, g);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          typename W::Raw raw;
+          W::load(raw, wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g,
+                  min(8, (a.K >> 5) - 8 * c));
+          add_large<W, 1>(reinterpret_cast<floatx4(&)[1]>(tot[r]), raw, lane,
+                          [&](int st, int, half8v& hi, half8v& lo) { hi = ah[st]; lo = al[st]; },
+                          [&](int) { return inv; });
+        }
+      }
     }
   }
   if constexpr (KW > 1) {
@@ -611,6 +729,16 @@ gemm_many_kernel(GemmArgs a) {
         hi = *reinterpret_cast<const half8v*>(at);
         lo = *reinterpret_cast<const half8v*>(at + 1024);
       };
+      if constexpr (W::kBlocks32) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          if (sc[r].large) [[unlikely]]
+            add_large<W, JT>(tot[r], raw[r], lane,
+                             [&](int st, int j, half8v& hi, half8v& lo) { operand(st * JT + j, hi, lo); },
+                             [&](int j) {
+                               return *reinterpret_cast<const floatx4*>(buf + L::kInv + 64 * j + 16 * g);
+                             });
+      }
       half8v ah[2], al[2], bh[RT], bl[RT];
       operand(0, ah[0], al[0]);
 #pragma unroll

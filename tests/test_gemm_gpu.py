@@ -120,6 +120,38 @@ def test_extreme_activations_and_scales(hip, type_tag):
         s.close()
 
 
+@pytest.mark.parametrize("type_tag", [ggml.Q5_0, ggml.Q8_0], ids=["Q5_0", "Q8_0"])
+@pytest.mark.parametrize("shape", [(40, 480, 3), (515, 1056, 16), (4000, 480, 65), (14000, 320, 63),
+                                   (14300, 256, 200)], ids=lambda s: "x".join(map(str, s)))
+def test_large_scales_leave_small_ones_exact(hip, type_tag, shape):
+    """Scales of 256 and more beside scales of 1e-5 to 1e-3: in another row of
+    the tile, and in another block of the same row where the large block's
+    weights are zero.  Each row is held to its own bound."""
+    rows, columns, tokens = shape
+    rng = np.random.default_rng(rows)
+    w = synthetic.packed(type_tag, rng, rows, columns)
+    blocks = w.reshape(rows, columns // 32, ggml.block_bytes(type_tag))
+    small = rng.choice(np.array([1e-3, 1e-4, -1e-5, 5e-6], dtype=np.float16), size=blocks.shape[:2])
+    blocks[:, :, 0:2] = small.view(np.uint8).reshape(*blocks.shape[:2], 2)
+    large = np.array([256.0, -2000.0, 65504.0], dtype=np.float16).view(np.uint8).reshape(3, 2)
+    zero = np.zeros(ggml.block_bytes(type_tag) - 2, dtype=np.uint8)
+    if type_tag == ggml.Q5_0:
+        zero[:4] = 0xFF  # fifth bits: code 16 is weight 0
+    for i, at in enumerate(range(0, rows, 16)):  # one row of each tile: one zero block of a large scale
+        r, b = at + i % min(16, rows - at), i % blocks.shape[1]
+        blocks[r, b, 0:2], blocks[r, b, 2:] = large[i % 3], zero
+        if i % 2:  # and every other tile a row of large scales among its own small ones
+            r = at + (i + 7) % min(16, rows - at)
+            blocks[r, ::3, 0:2] = large[i % 3]
+    x = synthetic.activations(rng, tokens, columns)
+    s = make_hip_session_packed(w, type_tag, rows, columns)
+    try:
+        y = _run(s, x)
+    finally:
+        s.close()
+    _check(type_tag, w, rows, columns, x, y, f"{ggml.NAMES[type_tag]} {shape}", norm=False)
+
+
 @pytest.mark.parametrize("shape", [(1, 4, 2), (33, 260, 16), (515, 1028, 17), (512, 2048, 33),
                                    (96, 4100, 130)], ids=lambda s: "x".join(map(str, s)))
 def test_f32_rows(hip, shape):
