@@ -965,27 +965,17 @@ static hipError_t launch_f32(const GemmArgs& a, bool one_order, hipStream_t stre
     return hipGetLastError();
   }
   const unsigned rows = (unsigned)((a.rows + 31) / 32);
-  // tokens in launches of at most 65535 tiles of 32
-  GemmArgs q = a;
-  for (int t0 = 0; t0 < a.tokens; t0 += 65535 * 32) {
-    q.tokens = std::min(65535 * 32, a.tokens - t0);
-    q.x = a.x + (int64_t)t0 * a.x_stride;
-    q.y = a.y + (int64_t)t0 * a.y_stride;
-    if (q.tokens <= 16)
-      hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3(rows), dim3(64 * kF32Waves), 0, stream, q);
-    else
-      hipLaunchKernelGGL(gemm_f32_kernel<2>, dim3(rows, (q.tokens + 31) / 32),
-                         dim3(64 * kF32Waves), 0, stream, q);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  if (a.tokens <= 16)
+    hipLaunchKernelGGL(gemm_f32_kernel<1>, dim3(rows), dim3(64 * kF32Waves), 0, stream, a);
+  else
+    hipLaunchKernelGGL(gemm_f32_kernel<2>, dim3(rows, (a.tokens + 31) / 32), dim3(64 * kF32Waves), 0,
+                       stream, a);
+  return hipGetLastError();
 }
 
 template <int TYPE, int RT, int KW>
 static hipError_t launch_few(const GemmArgs& a, hipStream_t stream) {
   const dim3 grid((a.rows + 16 * RT - 1) / (16 * RT), (a.tokens + 15) / 16);
-  if (grid.y > 65535) return hipErrorInvalidValue;  // never chosen: rounds make it the slowest
   hipLaunchKernelGGL((gemm_few_kernel<TYPE, RT, KW>), grid, dim3(64 * KW), 0, stream, a);
   return hipGetLastError();
 }
@@ -995,8 +985,7 @@ static hipError_t launch_many(const GemmArgs& a_in, hipStream_t stream) {
   GemmArgs a = a_in;
   a.row_tiles = (a.rows + 16 * RT * RW - 1) / (16 * RT * RW);
   a.token_tiles = (a.tokens + 16 * JT - 1) / (16 * JT);
-  const int64_t total = (int64_t)a.row_tiles * a.token_tiles;
-  if (total > (1 << 30)) return hipErrorInvalidValue;
+  const int total = a.row_tiles * a.token_tiles;
   constexpr int lds = KW * 2 * GemmLds<TYPE, JT>::kBytes;
   static_assert(lds <= (int)kMaxLdsBytes && (KW - 1) * RW * RT * JT * 1024 <= lds, "LDS");
   const auto kernel = gemm_many_kernel<TYPE, RT, JT, RW, KW>;
@@ -1051,6 +1040,17 @@ static hipError_t launch_type(const GemmArgs& a, bool one_order, hipStream_t str
   }
 }
 
+static hipError_t launch(int type, const GemmArgs& a, bool one_order, hipStream_t stream) {
+  switch (type) {
+    case kQ4_K: return launch_type<kQ4_K>(a, one_order, stream);
+    case kQ6_K: return launch_type<kQ6_K>(a, one_order, stream);
+    case kQ5_0: return launch_type<kQ5_0>(a, one_order, stream);
+    case kQ8_0: return launch_type<kQ8_0>(a, one_order, stream);
+    case kF32: return launch_f32(a, one_order, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream) {
   if (p.tokens < 1 || p.rows < 1 || p.rows > INT32_MAX || p.columns % block_weights(p.type))
     return hipErrorInvalidValue;
@@ -1061,25 +1061,28 @@ hipError_t gemm_launch(const GemvProblem& p, hipStream_t stream) {
   if (p.type == kF32 && p.columns % 4) return hipErrorInvalidValue;
   // lane offsets within a tile are 32 bits
   if (p.x_stride < 0 || p.x_stride > (1 << 22) || p.row_bytes > (1 << 22)) return hipErrorInvalidValue;
-  GemmArgs a{};
-  a.w = p.weights;
-  a.row_bytes = p.row_bytes;
-  a.rows = (int)p.rows;
-  a.K = (int)p.columns;
-  a.chunks = (a.K + 255) / 256;
-  a.x = p.x;
-  a.x_stride = p.x_stride;
-  a.tokens = p.tokens;
-  a.y = p.y;
-  a.y_stride = p.y_stride;
-  switch (p.type) {
-    case kQ4_K: return launch_type<kQ4_K>(a, p.one_order, stream);
-    case kQ6_K: return launch_type<kQ6_K>(a, p.one_order, stream);
-    case kQ5_0: return launch_type<kQ5_0>(a, p.one_order, stream);
-    case kQ8_0: return launch_type<kQ8_0>(a, p.one_order, stream);
-    case kF32: return launch_f32(a, p.one_order, stream);
-    default: return hipErrorInvalidValue;
-  }
+  // A grid has less than 2^32 threads and at most 65535 workgroups in its
+  // second dimension: launches of at most 2^20 rows and as many tokens as
+  // 2^22 tiles of 16 x 16, the smallest, hold (whole tiles of every shape)
+  const int64_t row_span = std::min<int64_t>(p.rows, 1 << 20), row_tiles = (row_span + 15) / 16;
+  const int64_t token_span = 64 * (std::min<int64_t>(65535, (1 << 22) / row_tiles) / 4);
+  for (int64_t r0 = 0; r0 < p.rows; r0 += row_span)
+    for (int64_t t0 = 0; t0 < p.tokens; t0 += token_span) {
+      GemmArgs a{};
+      a.w = p.weights + r0 * p.row_bytes;
+      a.row_bytes = p.row_bytes;
+      a.rows = (int)std::min(row_span, p.rows - r0);
+      a.K = (int)p.columns;
+      a.chunks = (a.K + 255) / 256;
+      a.x = p.x + t0 * p.x_stride;
+      a.x_stride = p.x_stride;
+      a.tokens = (int)std::min(token_span, p.tokens - t0);
+      a.y = p.y + t0 * p.y_stride + r0;
+      a.y_stride = p.y_stride;
+      const hipError_t e = launch(p.type, a, p.one_order, stream);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
 }
 
 }  // namespace llhip

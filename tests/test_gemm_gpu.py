@@ -174,6 +174,29 @@ def test_f32_rows(hip, shape):
     assert np.array_equal(*((first, y[:5]) if tokens > 4 else (again, y[:2])))
 
 
+@pytest.mark.parametrize("type_tag,rows,columns,tokens", [
+    (ggml.Q8_0, 16, 32, 16 * 65535 + 20), (ggml.Q5_0, (1 << 20) + 40, 32, 3),
+    (ggml.F32, (1 << 20) + 5, 4, 5), (ggml.F32, 7, 8, 16 * 65535 + 9)],
+    ids=lambda v: str(v))
+def test_more_rows_or_tokens_than_one_grid_takes(hip, type_tag, rows, columns, tokens):
+    import torch
+    rng = np.random.default_rng(9)
+    w = synthetic.packed(type_tag, rng, rows, columns)
+    x = synthetic.activations(rng, tokens, columns)
+    wd = torch.from_numpy(_weights(type_tag, w, rows, columns)).cuda()
+    xd = torch.from_numpy(x).cuda()
+    yd = torch.full((tokens, rows), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    s = make_hip_session_packed(w, type_tag, rows, columns)
+    try:
+        s.run_device(xd.data_ptr(), yd.data_ptr(), tokens)
+        torch.cuda.synchronize()
+    finally:
+        s.close()
+    bound = 2.0 ** -20 * (xd.double().abs() @ wd.abs().T.contiguous())
+    assert bool(((yd.double() - xd.double() @ wd.T.contiguous()).abs() <= bound).all())
+
+
 def test_device_rows_on_any_float(hip):
     """x and y need float alignment only; neighbours of y stay untouched."""
     import torch
