@@ -109,28 +109,25 @@ struct GemmW<kQ6_K> {
 
 // Scales of a 32-block type: d of blocks 2g and 2g + 1.  Blocks past the row's
 // end (the last chunk of a K that 256 does not divide) count 0.  A |d| of 256
-// or more would leave f16's range in d q: such blocks count 0 in a chunk's
-// products, and the wave adds them in a pass of their own, as d / 256 (d / 256
-// of the small d beside them would fall among f16's subnormals).
+// or more would leave f16's range in d q: a chunk that has one is multiplied
+// in two parts, the large scales as d / 256, each with the other part's blocks
+// at 0 (d / 256 of the small ones would fall among f16's subnormals).
 struct BlockScale {
   half2v sl, sh;
-  uint64_t large;  // lanes with a |d| of 256 or more
+  bool large;  // this lane has a |d| of 256 or more
   __device__ __forceinline__ void set(uint32_t d0, uint32_t d1, int g, int blocks) {
     d0 = 2 * g < blocks ? d0 & 0xFFFFu : 0u;
     d1 = 2 * g + 1 < blocks ? d1 & 0xFFFFu : 0u;
-    large = __ballot(is_large(d0) || is_large(d1));
-    d0 = is_large(d0) ? 0u : d0;
-    d1 = is_large(d1) ? 0u : d1;
+    large = is_large(d0) || is_large(d1);
     sl = as_half2(d0 | (d0 << 16));
     sh = as_half2(d1 | (d1 << 16));
   }
-  __device__ __forceinline__ void set_large(uint32_t d0, uint32_t d1, int g, int blocks) {
-    const half2v f = splat2((_Float16)(1.f / 256.f));
-    d0 = 2 * g < blocks && is_large(d0) ? d0 & 0xFFFFu : 0u;
-    d1 = 2 * g + 1 < blocks && is_large(d1) ? d1 & 0xFFFFu : 0u;
-    large = __ballot((d0 | d1) != 0u);
-    sl = as_half2(d0 | (d0 << 16)) * f;
-    sh = as_half2(d1 | (d1 << 16)) * f;
+  template <bool LARGE>
+  __device__ __forceinline__ void set_part(uint32_t d0, uint32_t d1, int g, int blocks) {
+    set(d0, d1, g, blocks);
+    const half2v f = splat2((_Float16)(LARGE ? 1.f / 256.f : 1.f));
+    sl = is_large(d0) == LARGE ? sl * f : splat2((_Float16)0.f);
+    sh = is_large(d1) == LARGE ? sh * f : splat2((_Float16)0.f);
   }
   static __device__ __forceinline__ bool is_large(uint32_t d) { return (d & 0x7FFFu) >= 0x5C00u; }
 };
@@ -160,8 +157,9 @@ struct GemmW<kQ8_0> : QuadsByGroup {
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[8] >> 16, g, r.blocks);
   }
-  static __device__ __forceinline__ void prepare_large(Scale& c, const Raw& r, int g) {
-    c.set_large(r.w[0], r.w[8] >> 16, g, r.blocks);
+  template <bool LARGE>
+  static __device__ __forceinline__ void prepare_part(Scale& c, const Raw& r, int g) {
+    c.set_part<LARGE>(r.w[0], r.w[8] >> 16, g, r.blocks);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
                                               int s) {
@@ -204,8 +202,9 @@ struct GemmW<kQ5_0> : QuadsByGroup {
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[5] >> 16, g, r.blocks);
   }
-  static __device__ __forceinline__ void prepare_large(Scale& c, const Raw& r, int g) {
-    c.set_large(r.w[0], r.w[5] >> 16, g, r.blocks);
+  template <bool LARGE>
+  static __device__ __forceinline__ void prepare_part(Scale& c, const Raw& r, int g) {
+    c.set_part<LARGE>(r.w[0], r.w[5] >> 16, g, r.blocks);
   }
   // element 4s + b: nibble s >> 2 of qs byte 4 (s & 3) + b, fifth bit 4s + b of qh
   static __device__ __forceinline__ uint32_t code(uint32_t qs, uint32_t qh, int s) {
@@ -244,19 +243,19 @@ struct GemmArgs {
   int row_tiles, token_tiles;  // gemm_many_kernel
 };
 
-// The large scales' products (BlockScale) of one row tile's chunk, JT token
-// tiles: operand(st, j, hi, lo) gives step st's activations of tile j.  Rows
-// without a large scale keep their totals (their products are 0 times x).
-template <typename W, int JT, typename Operand, typename Inverse>
-__device__ __forceinline__ void add_large(floatx4 (&tot)[JT], const typename W::Raw& raw,
-                                          int lane, Operand operand, Inverse inverse) {
+// One part's products (BlockScale) of one row tile's chunk and JT token tiles:
+// operand(st, j, hi, lo) gives step st's activations of tile j.  Rows without
+// a large scale keep their totals in the large part (0 times x).
+template <typename W, int JT, bool LARGE, typename Operand, typename Inverse>
+__device__ __forceinline__ void add_part(floatx4 (&tot)[JT], const typename W::Raw& raw, int lane,
+                                         Operand operand, Inverse inverse) {
   // the codes anew: shared with the chunk's other products they would be kept
   // in registers from here on
   typename W::Raw own = raw;
 #pragma unroll
   for (uint32_t& v : own.w) v = opaque(v);
   typename W::Scale sc;
-  W::prepare_large(sc, own, lane >> 4);
+  W::template prepare_part<LARGE>(sc, own, lane >> 4);
   floatx4 blk[JT];
 #pragma unroll
   for (int j = 0; j < JT; ++j) blk[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -274,14 +273,15 @@ __device__ __forceinline__ void add_large(floatx4 (&tot)[JT], const typename W::
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  const uint64_t m = sc.large;
+  const uint64_t m = __ballot(sc.large);
   const uint32_t rows = (uint32_t)(m | (m >> 16) | (m >> 32) | (m >> 48));
-  if ((rows >> (lane & 15)) & 1u) {
+  if (!LARGE || ((rows >> (lane & 15)) & 1u)) {
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
       const floatx4 inv = inverse(j);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) tot[j][i] = fmaf(256.f * inv[i], blk[j][i], tot[j][i]);
+      for (int i = 0; i < 4; ++i)
+        tot[j][i] = fmaf(LARGE ? 256.f * inv[i] : inv[i], blk[j][i], tot[j][i]);
     }
   }
 }
@@ -353,7 +353,7 @@ gemm_few_kernel(GemmArgs a) {
   floatx4 tot[RT];
 #pragma unroll
   for (int r = 0; r < RT; ++r) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
-  uint64_t large = 0;
+  bool large = false;  // 32-block types: a large scale among this lane's
 
   for (int c = kw; c < a.chunks; c += KW) {
     const int blocks = W::kBlocks32 ? min(8, (a.K >> 5) - 8 * c) : 8;
@@ -438,9 +438,11 @@ gemm_few_kernel(GemmArgs a) {
     }
   }
   if constexpr (W::kBlocks32) {
-    // the chunks again if any has a large scale (out of the loop above, whose
-    // one block of decode and products runs 2 to 5% longer with a branch in it)
-    if (large) [[unlikely]] {
+    // all anew in two parts if any chunk has a large scale (the loop above runs
+    // 2 to 5% longer with that branch, or the parts' selects, in it)
+    if (__any(large)) [[unlikely]] {
+#pragma unroll
+      for (int r = 0; r < RT; ++r) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
       for (int c = kw; c < a.chunks; c += KW) {
         half8v ah[8], al[8];
         floatx4 inv;
@@ -450,9 +452,11 @@ gemm_few_kernel(GemmArgs a) {
           typename W::Raw raw;
           W::load(raw, wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g,
                   min(8, (a.K >> 5) - 8 * c));
-          add_large<W, 1>(reinterpret_cast<floatx4(&)[1]>(tot[r]), raw, lane,
-                          [&](int st, int, half8v& hi, half8v& lo) { hi = ah[st]; lo = al[st]; },
-                          [&](int) { return inv; });
+          auto& one = reinterpret_cast<floatx4(&)[1]>(tot[r]);
+          const auto operand = [&](int st, int, half8v& hi, half8v& lo) { hi = ah[st]; lo = al[st]; };
+          const auto inverse = [&](int) { return inv; };
+          add_part<W, 1, false>(one, raw, lane, operand, inverse);
+          add_part<W, 1, true>(one, raw, lane, operand, inverse);
         }
       }
     }
@@ -715,7 +719,12 @@ gemm_many_kernel(GemmArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       typename W::Scale sc[RT];
 #pragma unroll
-      for (int r = 0; r < RT; ++r) W::prepare(sc[r], raw[r], g);
+      for (int r = 0; r < RT; ++r) {
+        if constexpr (W::kBlocks32)
+          W::template prepare_part<false>(sc[r], raw[r], g);
+        else
+          W::prepare(sc[r], raw[r], g);
+      }
       // the small products have sums of their own where registers allow: each
       // add rounds in proportion to the sum it meets
       constexpr bool kOwnLo = RT * JT <= 8;
@@ -732,12 +741,12 @@ gemm_many_kernel(GemmArgs a) {
       if constexpr (W::kBlocks32) {
 #pragma unroll
         for (int r = 0; r < RT; ++r)
-          if (sc[r].large) [[unlikely]]
-            add_large<W, JT>(tot[r], raw[r], lane,
-                             [&](int st, int j, half8v& hi, half8v& lo) { operand(st * JT + j, hi, lo); },
-                             [&](int j) {
-                               return *reinterpret_cast<const floatx4*>(buf + L::kInv + 64 * j + 16 * g);
-                             });
+          if (__any(sc[r].large)) [[unlikely]]
+            add_part<W, JT, true>(tot[r], raw[r], lane,
+                                  [&](int st, int j, half8v& hi, half8v& lo) { operand(st * JT + j, hi, lo); },
+                                  [&](int j) {
+                                    return *reinterpret_cast<const floatx4*>(buf + L::kInv + 64 * j + 16 * g);
+                                  });
       }
       half8v ah[2], al[2], bh[RT], bl[RT];
       operand(0, ah[0], al[0]);

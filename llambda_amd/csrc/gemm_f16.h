@@ -19,7 +19,7 @@
 //               the remainder (exact); d once per chunk
 //   Q5_0, Q8_0  d * q, at most 18 bits, as hi + lo (exact: every product is
 //               a multiple of 2^-24, f16's smallest step).  Blocks with a
-//               |d| of 256 or more are multiplied in a pass of their own, as
+//               |d| of 256 or more are multiplied in a part of their own, as
 //               d / 256
 // Products accumulate in fp32 over the chunk on v_mfma_f32_16x16x32_f16:
 // (x hi + x lo) against one f16, or the three products hi hi + lo hi + hi lo
