@@ -431,7 +431,13 @@ gemm_few_kernel(GemmArgs a) {
         if constexpr (W::kPair) blk = mfma_f16(ah[st], bl, blk);
       }
 #pragma unroll
-      for (int st = 0; st < 8; ++st) blk = mfma_f16(ah[st], bh[st], blk);
+      for (int st = 0; st < (W::kMin ? 4 : 8); ++st) blk = mfma_f16(ah[st], bh[st], blk);
+      if constexpr (W::kMin) {
+        floatx4 half = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 4; st < 8; ++st) half = mfma_f16(ah[st], bh[st], half);
+        blk += half;
+      }
       typename W::Finish fin;
       W::finish(fin, raw[r], sc, g);
       add_products<W>(tot[r], blk, inv, fin, sums);
@@ -539,7 +545,7 @@ gemm_many_kernel(GemmArgs a) {
   constexpr int P = 4 * JT / RW;  // groups of four tokens a wave splits
   static_assert(P * RW == 4 * JT, "token groups");
   extern __shared__ __align__(16) uint8_t smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rw = wave % RW, kw = wave / RW;
   const int n = lane & 15, g = lane >> 4;
   uint8_t* lds = smem + kw * 2 * L::kBytes;
@@ -591,7 +597,7 @@ gemm_many_kernel(GemmArgs a) {
       for (int q = 0; q < 4; ++q)
         v[p][q] = (!W::kBlocks32 || 256 * c + 64 * q + 4 * n < a.K)
                       ? (floatx4)*reinterpret_cast<const floatx4a4*>(
-                            reinterpret_cast<const uint8_t*>(xbase + 256 * c) + (xoff[p] + 256u * q))
+                            reinterpret_cast<const uint8_t*>(xbase + 256 * c + 64 * q) + xoff[p])
                       : floatx4{0.f, 0.f, 0.f, 0.f};
   };
   auto split_x = [&](uint8_t* buf) {
@@ -729,6 +735,7 @@ gemm_many_kernel(GemmArgs a) {
       // add rounds in proportion to the sum it meets
       constexpr bool kOwnLo = RT * JT <= 8;
       floatx4 blk[RT][JT], low[kOwnLo ? RT : 1][kOwnLo ? JT : 1];
+      floatx4 half[W::kMin ? RT : 1][W::kMin ? JT : 1];  // Q4_K: the first steps' hi products
       const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
       // operand i = (step i / JT, token tile i % JT), read one ahead
       const uint32_t unit = opaque((uint32_t)lane);
@@ -765,9 +772,13 @@ gemm_many_kernel(GemmArgs a) {
         if constexpr (W::kPair)
 #pragma unroll
           for (int r = 0; r < RT; ++r) low_sum(r) = mfma_f16(h, bl[r], low_sum(r));
+        if constexpr (W::kMin)
+          if (st == 4)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) half[r][j] = blk[r][j];
 #pragma unroll
         for (int r = 0; r < RT; ++r)
-          blk[r][j] = mfma_f16(h, bh[r], kOwnLo && st == 0 ? zero : blk[r][j]);
+          blk[r][j] = mfma_f16(h, bh[r], (kOwnLo && st == 0) || (W::kMin && st == 4) ? zero : blk[r][j]);
         if (j == JT - 1) __builtin_amdgcn_sched_barrier(0);
       }
       typename W::Finish fin[RT];
@@ -786,6 +797,7 @@ gemm_many_kernel(GemmArgs a) {
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
           if constexpr (kOwnLo) blk[r][j] += low[r][j];
+          if constexpr (W::kMin) blk[r][j] += half[r][j];
           add_products<W>(tot[r][j], blk[r][j], inv, fin[r], sums);
         }
         __builtin_amdgcn_sched_barrier(0);

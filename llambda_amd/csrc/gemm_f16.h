@@ -8,13 +8,18 @@
 // brings the token's largest magnitude of the chunk into [2^14, 2^15): no
 // value overflows, and what subnormal lo parts lose is below 2^-39 of that
 // largest value.  A weight enters as an exact f16 integer or an exact pair:
-//   Q4_K        sc * (q - 8), at most 504: one f16; the chunk's d is applied
-//               once, to the chunk's sums.  The sub-blocks' offsets 8 sc and
-//               minima m ride in two extra products per chunk, against the
-//               sub-blocks' sums of x s / 32 (hi and lo).  The codes are
-//               centred because each add to the sums rounds in proportion to
-//               them (with sc * q the error against 64 bits was 1.75e-7, above
-//               the 1.2e-7 of an fp32 evaluation)
+//   Q4_K        sc * q, at most 945: one f16; the chunk's d is applied once, to
+//               the chunk's sums.  The sub-blocks' minima m ride in an extra
+//               product per chunk, against the sub-blocks' sums of x s / 32 (hi
+//               and lo).  Each add to the sums rounds in proportion to what
+//               they have reached, so the hi products of a chunk run in two
+//               halves (in one run the error against 64 bits of N(0, 1) tokens
+//               was 1.36e-7, an fp32 evaluation's 1.17e-7; in halves 1.15e-7).
+//               The expert products (moe_f16.h) keep one run and centre the
+//               codes, sc * (q - 8), with the offsets 8 sc in a second extra
+//               product: as exact on such tokens, but an activation 2^13 times
+//               the others leaves the rows with the smallest weights for it up
+//               to eight times as far off
 //   Q6_K        sc * (q - 32), 13 bits: hi = the product rounded to f16, lo =
 //               the remainder (exact); d once per chunk
 //   Q5_0, Q8_0  d * q, at most 18 bits, as hi + lo (exact: every product is
@@ -59,6 +64,13 @@ __device__ __forceinline__ half2v bytes02(uint32_t v) {
 __device__ __forceinline__ half2v bytes13(uint32_t v) {
   return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u));
 }
+// The same as f16 byte * 2^-24.
+__device__ __forceinline__ half2v subnormal02(uint32_t v) {
+  return as_half2(__builtin_amdgcn_perm(v, v, 0x0C020C00u));
+}
+__device__ __forceinline__ half2v subnormal13(uint32_t v) {
+  return as_half2(__builtin_amdgcn_perm(v, v, 0x0C030C01u));
+}
 __device__ __forceinline__ half8v join8(half2v a, half2v b, half2v c, half2v d) {
   return half8v{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
 }
@@ -89,21 +101,12 @@ struct QuadsByGroup {
   static constexpr int quarter_bytes(int q) { return 256 * q; }
 };
 
-template <>
-struct GemmW<kQ4_K> : QuadsByGroup {
+// Q4_K rows: the chunk's bytes and the decode of its scales and minima.
+struct Q4KRow : QuadsByGroup {
   static constexpr int kBytes = 144;
   static constexpr bool kPair = false, kMin = true, kBlocks32 = false;
   struct Raw {
     uint4 h, q0, q1;
-  };
-  struct Scale {
-    half2v sl, ol, sh, oh;  // sc / 16 and -72 sc of sub-blocks 2g and 2g + 1
-  };
-  struct Finish {
-    // against ChunkSums: the f16 pairs {m, m} of both sub-blocks and {m0, m1};
-    // the same of 256 sc (8 sc S = 256 sc S / 32)
-    uint32_t m0, m1, m2, c0, c1, c2;
-    float d, dm;  // d and -32 dmin
   };
   // the 16-byte header and qs bytes [32 g, 32 g + 32); 16-byte aligned rows
   static __device__ __forceinline__ void load(Raw& r, const uint8_t* b, uint32_t o, int g, int) {
@@ -114,44 +117,62 @@ struct GemmW<kQ4_K> : QuadsByGroup {
   }
   // get-scale-min-k4-at (llambda.lisp:4316-4336) of sub-blocks 2g, 2g + 1
   // (both at once, in bytes 0 and 1)
-  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+  static __device__ __forceinline__ uint32_t scale_bytes(const Raw& r, int g) {
     const int shift = 8 * ((2 * g) & 3);
     const uint32_t b0 = r.h.y >> shift, b8 = r.h.w >> shift;
-    const uint32_t sc = g >= 2 ? (b8 & 0x0F0Fu) | ((b0 >> 2) & 0x3030u) : b0 & 0x3F3Fu;
-    const half2v k1152 = splat2((_Float16)-1152.f);
-    c.sl = splat2((_Float16)((float)(sc & 0xFFu) * 0.0625f));
-    c.sh = splat2((_Float16)((float)((sc >> 8) & 0xFFu) * 0.0625f));
-    c.ol = c.sl * k1152;
-    c.oh = c.sh * k1152;
+    return g >= 2 ? (b8 & 0x0F0Fu) | ((b0 >> 2) & 0x3030u) : b0 & 0x3F3Fu;
   }
-  static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale& c, int g) {
+  static __device__ __forceinline__ uint32_t min_bytes(const Raw& r, int g) {
     const int shift = 8 * ((2 * g) & 3);
     const uint32_t b4 = r.h.z >> shift, b8 = r.h.w >> shift;
-    const uint32_t mn = g >= 2 ? ((b8 >> 4) & 0x0F0Fu) | ((b4 >> 2) & 0x3030u) : b4 & 0x3F3Fu;
-    const half2v m0 = splat2((_Float16)(float)(mn & 0xFFu));
-    const half2v m1 = splat2((_Float16)(float)((mn >> 8) & 0xFFu));
-    const half2v k4096 = splat2((_Float16)4096.f);
-    const half2v c0 = c.sl * k4096, c1 = c.sh * k4096;
-    f.m0 = __builtin_bit_cast(uint32_t, m0);
-    f.m1 = __builtin_bit_cast(uint32_t, m1);
-    f.m2 = __builtin_bit_cast(uint32_t, half2v{m0.x, m1.x});
-    f.c0 = __builtin_bit_cast(uint32_t, c0);
-    f.c1 = __builtin_bit_cast(uint32_t, c1);
-    f.c2 = __builtin_bit_cast(uint32_t, half2v{c0.x, c1.x});
-    f.d = half_bits_to_float(r.h.x & 0xFFFFu);
-    f.dm = -32.f * half_bits_to_float(r.h.x >> 16);
+    return g >= 2 ? ((b8 >> 4) & 0x0F0Fu) | ((b4 >> 2) & 0x3030u) : b4 & 0x3F3Fu;
   }
-  // sc (q - 8) = (1024 + 16 q) sc / 16 - 72 sc, exact in one fma
-  static __device__ __forceinline__ void frag(half8v& hi, half8v&, const Raw& r, const Scale& c,
-                                              int s) {
+  // the minima as f16 pairs {m, m} of both sub-blocks and {m0, m1}
+  static __device__ __forceinline__ void minima(uint32_t mn, uint32_t& m0, uint32_t& m1,
+                                                uint32_t& m2) {
+    const half2v a = splat2((_Float16)(float)(mn & 0xFFu));
+    const half2v b = splat2((_Float16)(float)((mn >> 8) & 0xFFu));
+    m0 = __builtin_bit_cast(uint32_t, a);
+    m1 = __builtin_bit_cast(uint32_t, b);
+    m2 = __builtin_bit_cast(uint32_t, half2v{a.x, b.x});
+  }
+  // the dword of step s's codes: low and high nibbles
+  static __device__ __forceinline__ uint32_t codes(const Raw& r, int s) {
     const uint4 v = s < 4 ? r.q0 : r.q1;
     const int i = s & 3;
-    const uint32_t w = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-    const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hg = w & 0xF0F0F0F0u;
-    hi = join8(__builtin_elementwise_fma(bytes02(lo), c.sl, c.ol),
-               __builtin_elementwise_fma(bytes13(lo), c.sl, c.ol),
-               __builtin_elementwise_fma(bytes02(hg), c.sh, c.oh),
-               __builtin_elementwise_fma(bytes13(hg), c.sh, c.oh));
+    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+  }
+};
+
+template <>
+struct GemmW<kQ4_K> : Q4KRow {
+  static constexpr bool kCentred = false;
+  struct Scale {
+    half2v sl, sh;  // 2^10 sc of sub-block 2g, 2^6 sc of 2g + 1
+    uint32_t mn;
+  };
+  struct Finish {
+    uint32_t m0, m1, m2;  // against the sub-blocks' sums
+    float d, dm;          // 2^14 d and -32 dmin
+  };
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    const uint32_t sc = scale_bytes(r, g);
+    c.sl = splat2((_Float16)((float)(sc & 0xFFu) * 1024.f));
+    c.sh = splat2((_Float16)((float)((sc >> 8) & 0xFFu) * 64.f));
+    c.mn = min_bytes(r, g);
+  }
+  static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale& c, int) {
+    minima(c.mn, f.m0, f.m1, f.m2);
+    f.d = 16384.f * half_bits_to_float(r.h.x & 0xFFFFu);
+    f.dm = -32.f * half_bits_to_float(r.h.x >> 16);
+  }
+  // 2^-14 sc q = (q 2^-24) (2^10 sc) = (16 q 2^-24) (2^6 sc): a nibble where it
+  // lies in its byte is an f16 subnormal
+  static __device__ __forceinline__ void frag(half8v& hi, half8v&, const Raw& r, const Scale& c,
+                                              int s) {
+    const uint32_t w = codes(r, s), lo = w & 0x0F0F0F0Fu, hg = w & 0xF0F0F0F0u;
+    hi = join8(subnormal02(lo) * c.sl, subnormal13(lo) * c.sl, subnormal02(hg) * c.sh,
+               subnormal13(hg) * c.sh);
   }
 };
 
@@ -221,9 +242,10 @@ __device__ __forceinline__ void add_products(floatx4& tot, const floatx4& blk, c
   if constexpr (W::kMin) {
     const half8v a = __builtin_bit_cast(half8v, sums);
     const half8v m = __builtin_bit_cast(half8v, u32x4{c.m0, c.m1, c.m2, 0u});
-    const half8v o = __builtin_bit_cast(half8v, u32x4{c.c0, c.c1, c.c2, 0u});
     const floatx4 mn = mfma_f16(a, m, floatx4{0.f, 0.f, 0.f, 0.f});
-    const floatx4 all = mfma_f16(a, o, blk);
+    floatx4 all = blk;
+    if constexpr (W::kCentred)
+      all = mfma_f16(a, __builtin_bit_cast(half8v, u32x4{c.c0, c.c1, c.c2, 0u}), blk);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       tot[i] = fmaf(inv[i], fmaf(c.d, all[i], c.dm * mn[i]), tot[i]);

@@ -12,13 +12,50 @@ namespace llhip {
 template <int TYPE>
 struct ExpertW;
 
+// Codes centred (gemm_f16.h).
 template <>
-struct ExpertW<kQ4_K> : GemmW<kQ4_K> {
+struct ExpertW<kQ4_K> : Q4KRow {
   static constexpr int kPitch = 144;
+  static constexpr bool kCentred = true;
+  struct Scale {
+    half2v sl, ol, sh, oh;  // sc / 16 and -72 sc of sub-blocks 2g and 2g + 1
+  };
+  struct Finish {
+    uint32_t m0, m1, m2, c0, c1, c2;  // against the sub-blocks' sums: minima, and 256 sc
+    float d, dm;                      // d and -32 dmin
+  };
   static __device__ __forceinline__ void place(int i, int& g, int& s, int& high) {
     g = i >> 4;
     s = i & 7;
     high = (i >> 3) & 1;
+  }
+  static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
+    const uint32_t sc = scale_bytes(r, g);
+    const half2v k1152 = splat2((_Float16)-1152.f);
+    c.sl = splat2((_Float16)((float)(sc & 0xFFu) * 0.0625f));
+    c.sh = splat2((_Float16)((float)((sc >> 8) & 0xFFu) * 0.0625f));
+    c.ol = c.sl * k1152;
+    c.oh = c.sh * k1152;
+  }
+  static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale& c, int g) {
+    minima(min_bytes(r, g), f.m0, f.m1, f.m2);
+    // (8 sc S = 256 sc S / 32)
+    const half2v k4096 = splat2((_Float16)4096.f);
+    const half2v c0 = c.sl * k4096, c1 = c.sh * k4096;
+    f.c0 = __builtin_bit_cast(uint32_t, c0);
+    f.c1 = __builtin_bit_cast(uint32_t, c1);
+    f.c2 = __builtin_bit_cast(uint32_t, half2v{c0.x, c1.x});
+    f.d = half_bits_to_float(r.h.x & 0xFFFFu);
+    f.dm = -32.f * half_bits_to_float(r.h.x >> 16);
+  }
+  // sc (q - 8) = (1024 + 16 q) sc / 16 - 72 sc, exact in one fma
+  static __device__ __forceinline__ void frag(half8v& hi, half8v&, const Raw& r, const Scale& c,
+                                              int s) {
+    const uint32_t w = codes(r, s), lo = (w << 4) & 0xF0F0F0F0u, hg = w & 0xF0F0F0F0u;
+    hi = join8(__builtin_elementwise_fma(bytes02(lo), c.sl, c.ol),
+               __builtin_elementwise_fma(bytes13(lo), c.sl, c.ol),
+               __builtin_elementwise_fma(bytes02(hg), c.sh, c.oh),
+               __builtin_elementwise_fma(bytes13(hg), c.sh, c.oh));
   }
 };
 

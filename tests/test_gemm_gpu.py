@@ -5,8 +5,9 @@ Bounds.  Every output's error is at most 2^-20 of its sum of |terms|: the
 activations carry 2^-23 relative error, and the longest run of fp32 adds into
 one sum is 8 chunks x (about 40 roundings in a chunk) with partial sums below
 the sum of |terms|, whose roundings add up at random (sqrt(320) 2^-24 < 2^-19,
-and the partial sums average half of the bound).  A Q4_K term counts as the
-three products it is formed from: sc (q - 8) d, 8 sc d and m dmin.  The 2-norm
+and the partial sums average half of the bound).  A Q4_K term counts as
+three products, sc (q - 8) d, 8 sc d and m dmin, more than the two it is formed
+from (test_one_large_activation takes these two).  The 2-norm
 error of N(0, 1) activations stays below 3e-7 (an fp32 evaluation: 1.2e-7 to
 2.4e-7).
 """
@@ -150,6 +151,42 @@ def test_large_scales_leave_small_ones_exact(hip, type_tag, shape):
     finally:
         s.close()
     _check(type_tag, w, rows, columns, x, y, f"{ggml.NAMES[type_tag]} {shape}", norm=False)
+
+
+@pytest.mark.parametrize("shape", [(40, 512, 3), (515, 2048, 16), (4000, 768, 65), (1024, 2560, 33),
+                                   (14300, 256, 200)], ids=lambda s: "x".join(map(str, s)))
+def test_one_large_activation(hip, shape):
+    """An activation 2^22 times the others leaves its hold on the rows where its
+    Q4_K weight is zero (code and minimum) at what the split of x loses beside
+    it: 2^-39 of it per activation of its 256, whose lo parts are f16 subnormals
+    then.  Otherwise each row is held to 2^-20 of the products it is formed
+    from, sc q d and m dmin."""
+    rows, columns, tokens = shape
+    rng = np.random.default_rng(rows)
+    w = synthetic.packed(ggml.Q4_K, rng, rows, columns)
+    b = w.reshape(rows, columns // 256, 144)
+    at = 256 * (columns // 256 // 2) + 100  # sub-block 3 of a chunk: high nibbles of qs[32:64]
+    zeroed = b[::2, at // 256]
+    zeroed[:, 11] &= 0xC0  # its minimum
+    zeroed[:, 52] &= 0x0F  # the element's code
+    x = synthetic.activations(rng, tokens, columns)
+    x[:, at] = np.float32(2.0 ** 22)
+    s = make_hip_session_packed(w, ggml.Q4_K, rows, columns)
+    try:
+        y = _run(s, x)
+    finally:
+        s.close()
+    wd = _weights(ggml.Q4_K, w, rows, columns)
+    assert not wd[::2, at].any()
+    m = np.concatenate([b[:, :, 8:12] & 63, (b[:, :, 12:16] >> 4) | (b[:, :, 8:12] >> 6 << 4)], axis=2)
+    low = b[:, :, 2:4].copy().view(np.float16).astype(np.float64) * m
+    low = np.repeat(np.abs(low), 32, axis=2).reshape(rows, columns)
+    x = x.astype(np.float64)
+    terms = np.abs(wd + low) + low
+    chunk = slice(at // 256 * 256, at // 256 * 256 + 256)
+    bound = 2.0 ** -20 * (np.abs(x) @ terms.T) + 2.0 ** (22 - 39) * terms[:, chunk].sum(axis=1)
+    err = np.abs(y - x @ wd.T)
+    assert np.all(err <= bound), float((err / bound).max())
 
 
 @pytest.mark.parametrize("shape", [(1, 4, 2), (33, 260, 16), (515, 1028, 17), (512, 2048, 33),
