@@ -10,6 +10,11 @@
 
 namespace llhip {
 
+// v_mul_u32_u24 (a plain product becomes a v_mul_lo_u32 here, at a quarter of
+// the rate; written in inline asm it would get no wait states after an MFMA
+// whose result lies in its register).
+extern "C" __device__ uint32_t mul_u24(uint32_t a, uint32_t b) __asm("llvm.amdgcn.mul.u24.i32");
+
 // Rows that start on any even byte: b moves down to its dword, and the dword
 // at or below the old b + o is at the returned offset from it, `shift` bytes
 // below.  (The offset is formed from the dword base, so it never goes below
@@ -109,9 +114,9 @@ struct GemmW<kQ6_K> {
 
 // Scales of a 32-block type: d of blocks 2g and 2g + 1.  Blocks past the row's
 // end (the last chunk of a K that 256 does not divide) count 0.  A |d| of 256
-// or more would leave f16's range in d q: a chunk that has one is multiplied
-// in two parts, the large scales as d / 256, each with the other part's blocks
-// at 0 (d / 256 of the small ones would fall among f16's subnormals).
+// or more would leave f16's range in d q: a wave that meets one forms its sums
+// anew in two parts, the large scales as d / 256, each with the other part's
+// blocks at 0 (d / 256 of the small ones would fall among f16's subnormals).
 struct BlockScale {
   half2v sl, sh;
   bool large;  // this lane has a |d| of 256 or more
@@ -122,12 +127,11 @@ struct BlockScale {
     sl = as_half2(d0 | (d0 << 16));
     sh = as_half2(d1 | (d1 << 16));
   }
-  template <bool LARGE>
-  __device__ __forceinline__ void set_part(uint32_t d0, uint32_t d1, int g, int blocks) {
+  __device__ __forceinline__ void set_part(bool part, uint32_t d0, uint32_t d1, int g, int blocks) {
     set(d0, d1, g, blocks);
-    const half2v f = splat2((_Float16)(LARGE ? 1.f / 256.f : 1.f));
-    sl = is_large(d0) == LARGE ? sl * f : splat2((_Float16)0.f);
-    sh = is_large(d1) == LARGE ? sh * f : splat2((_Float16)0.f);
+    const half2v f = splat2((_Float16)(part ? 1.f / 256.f : 1.f));
+    sl = is_large(d0) == part ? sl * f : splat2((_Float16)0.f);
+    sh = is_large(d1) == part ? sh * f : splat2((_Float16)0.f);
   }
   static __device__ __forceinline__ bool is_large(uint32_t d) { return (d & 0x7FFFu) >= 0x5C00u; }
 };
@@ -157,9 +161,8 @@ struct GemmW<kQ8_0> : QuadsByGroup {
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[8] >> 16, g, r.blocks);
   }
-  template <bool LARGE>
-  static __device__ __forceinline__ void prepare_part(Scale& c, const Raw& r, int g) {
-    c.set_part<LARGE>(r.w[0], r.w[8] >> 16, g, r.blocks);
+  static __device__ __forceinline__ void prepare_part(bool part, Scale& c, const Raw& r, int g) {
+    c.set_part(part, r.w[0], r.w[8] >> 16, g, r.blocks);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
                                               int s) {
@@ -202,15 +205,13 @@ struct GemmW<kQ5_0> : QuadsByGroup {
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int g) {
     c.set(r.w[0], r.w[5] >> 16, g, r.blocks);
   }
-  template <bool LARGE>
-  static __device__ __forceinline__ void prepare_part(Scale& c, const Raw& r, int g) {
-    c.set_part<LARGE>(r.w[0], r.w[5] >> 16, g, r.blocks);
+  static __device__ __forceinline__ void prepare_part(bool part, Scale& c, const Raw& r, int g) {
+    c.set_part(part, r.w[0], r.w[5] >> 16, g, r.blocks);
   }
   // element 4s + b: nibble s >> 2 of qs byte 4 (s & 3) + b, fifth bit 4s + b of qh
   static __device__ __forceinline__ uint32_t code(uint32_t qs, uint32_t qh, int s) {
     const uint32_t n = s < 4 ? qs & 0x0F0F0F0Fu : (qs >> 4) & 0x0F0F0F0Fu;
-    uint32_t bits;  // bit i of the nibble to bit 8 i
-    asm("v_mul_u32_u24 %0, 0x204081, %1" : "=v"(bits) : "v"((qh >> (4 * s)) & 0xFu));
+    const uint32_t bits = mul_u24((qh >> (4 * s)) & 0xFu, 0x204081u);  // bit i of the nibble to bit 8 i
     return n | ((bits & 0x01010101u) << 4);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
@@ -231,6 +232,7 @@ struct GemmW<kQ5_0> : QuadsByGroup {
   }
 };
 
+
 struct GemmArgs {
   const uint8_t* w;
   int64_t row_bytes;
@@ -242,49 +244,6 @@ struct GemmArgs {
   int64_t y_stride;
   int row_tiles, token_tiles;  // gemm_many_kernel
 };
-
-// One part's products (BlockScale) of one row tile's chunk and JT token tiles:
-// operand(st, j, hi, lo) gives step st's activations of tile j.  Rows without
-// a large scale keep their totals in the large part (0 times x).
-template <typename W, int JT, bool LARGE, typename Operand, typename Inverse>
-__device__ __forceinline__ void add_part(floatx4 (&tot)[JT], const typename W::Raw& raw, int lane,
-                                         Operand operand, Inverse inverse) {
-  // the codes anew: shared with the chunk's other products they would be kept
-  // in registers from here on
-  typename W::Raw own = raw;
-#pragma unroll
-  for (uint32_t& v : own.w) v = opaque(v);
-  typename W::Scale sc;
-  W::template prepare_part<LARGE>(sc, own, lane >> 4);
-  floatx4 blk[JT];
-#pragma unroll
-  for (int j = 0; j < JT; ++j) blk[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int st = 0; st < 8; ++st) {
-    half8v bh, bl;
-    W::frag(bh, bl, own, sc, st);
-#pragma unroll
-    for (int j = 0; j < JT; ++j) {
-      half8v hi, lo;
-      operand(st, j, hi, lo);
-      blk[j] = mfma_f16(lo, bh, blk[j]);
-      blk[j] = mfma_f16(hi, bl, blk[j]);
-      blk[j] = mfma_f16(hi, bh, blk[j]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  const uint64_t m = __ballot(sc.large);
-  const uint32_t rows = (uint32_t)(m | (m >> 16) | (m >> 32) | (m >> 48));
-  if (!LARGE || ((rows >> (lane & 15)) & 1u)) {
-#pragma unroll
-    for (int j = 0; j < JT; ++j) {
-      const floatx4 inv = inverse(j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        tot[j][i] = fmaf(LARGE ? 256.f * inv[i] : inv[i], blk[j][i], tot[j][i]);
-    }
-  }
-}
 
 // The activations of lane (token n, group g) in chunk c, xr the token's row:
 // split into ah and al, with 1 / s of the tokens of D's rows in inv.
@@ -326,6 +285,64 @@ __device__ __forceinline__ void split_tokens(half8v (&ah)[8], half8v (&al)[8], f
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) inv[i] = __shfl(inv1, 4 * g + i);
+}
+
+// A wave's sums of RT row tiles and JT token tiles over chunks first, first +
+// step, ... in two parts (BlockScale), its operands straight from memory.  Rows
+// without a large scale keep their sums in the large part (0 times x).
+template <typename W, int RT, int JT>
+__device__ __forceinline__ void sum_in_parts(floatx4 (&tot)[RT][JT], const GemmArgs& a,
+                                             const uint8_t* wbase, const uint32_t (&woff)[RT],
+                                             int tok0, int first, int step, int lane) {
+  const int n = lane & 15, g = lane >> 4;
+#pragma unroll 1
+  for (int j = 0; j < JT; ++j) {
+    const float* xr = a.x + (int64_t)min(tok0 + 16 * j + n, a.tokens - 1) * a.x_stride;
+    floatx4 sum[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) sum[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = first; c < a.chunks; c += step) {
+      half8v ah[8], al[8];
+      floatx4 inv;
+      split_tokens<W>(ah, al, inv, xr, c, a.K, g);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        typename W::Raw raw;
+        W::load(raw, wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g,
+                min(8, (a.K >> 5) - 8 * c));
+#pragma unroll 1
+        for (int part = 0; part < 2; ++part) {
+          typename W::Scale sc;
+          W::prepare_part(part, sc, raw, g);
+          floatx4 blk = {0.f, 0.f, 0.f, 0.f};
+          half8v bh[8], bl;
+#pragma unroll
+          for (int st = 0; st < 8; ++st) {
+            W::frag(bh[st], bl, raw, sc, st);
+            blk = mfma_f16(al[st], bh[st], blk);
+            blk = mfma_f16(ah[st], bl, blk);
+          }
+#pragma unroll
+          for (int st = 0; st < 8; ++st) blk = mfma_f16(ah[st], bh[st], blk);
+          const uint64_t m = __ballot(sc.large);
+          const uint32_t rows = (uint32_t)(m | (m >> 16) | (m >> 32) | (m >> 48));
+          if (part == 0 || ((rows >> n) & 1u)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              sum[r][i] = fmaf(part ? 256.f * inv[i] : inv[i], blk[i], sum[r][i]);
+          }
+        }
+      }
+    }
+    // tile j's sums end up in tot[.][j] after the last turn
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+      for (int i = 0; i + 1 < JT; ++i) tot[r][i] = tot[r][i + 1];
+      tot[r][JT - 1] = sum[r];
+    }
+  }
 }
 
 // --------------------------------------------------------- few tokens
@@ -444,28 +461,10 @@ gemm_few_kernel(GemmArgs a) {
     }
   }
   if constexpr (W::kBlocks32) {
-    // all anew in two parts if any chunk has a large scale (the loop above runs
-    // 2 to 5% longer with that branch, or the parts' selects, in it)
-    if (__any(large)) [[unlikely]] {
-#pragma unroll
-      for (int r = 0; r < RT; ++r) tot[r] = floatx4{0.f, 0.f, 0.f, 0.f};
-      for (int c = kw; c < a.chunks; c += KW) {
-        half8v ah[8], al[8];
-        floatx4 inv;
-        split_tokens<W>(ah, al, inv, xr, c, a.K, g);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          typename W::Raw raw;
-          W::load(raw, wbase + (uint32_t)c * (uint32_t)W::kBytes, woff[r], g,
-                  min(8, (a.K >> 5) - 8 * c));
-          auto& one = reinterpret_cast<floatx4(&)[1]>(tot[r]);
-          const auto operand = [&](int st, int, half8v& hi, half8v& lo) { hi = ah[st]; lo = al[st]; };
-          const auto inverse = [&](int) { return inv; };
-          add_part<W, 1, false>(one, raw, lane, operand, inverse);
-          add_part<W, 1, true>(one, raw, lane, operand, inverse);
-        }
-      }
-    }
+    // (out of the loop above, which runs 2 to 5% longer with that branch or the
+    // parts' selects in it)
+    if (__any(large)) [[unlikely]]
+      sum_in_parts<W, RT, 1>(reinterpret_cast<floatx4(&)[RT][1]>(tot), a, wbase, woff, tok0, kw, KW, lane);
   }
   if constexpr (KW > 1) {
     if (kw > 0) {
@@ -473,14 +472,12 @@ gemm_few_kernel(GemmArgs a) {
       for (int r = 0; r < RT; ++r) red[kw - 1][r][lane] = tot[r];
     }
     __syncthreads();
-    // wave w adds row tiles w, w + KW, ... in wave order
+    if (kw != 0) return;
+    // the first wave adds them, in wave order
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      if (kw != 0) break;
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int q = 0; q < KW - 1; ++q) tot[r] += red[q][r][lane];
-    }
-    if (kw != 0) return;
   }
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
@@ -710,6 +707,7 @@ gemm_many_kernel(GemmArgs a) {
   constexpr int kSegment = 8;
 
   const int iters = (a.chunks + KW - 1) / KW;
+  bool large = false;  // 32-block types: a large scale among this lane's
   if (kw < a.chunks) {
     load_rows(kw);
     load_x(kw);
@@ -726,10 +724,8 @@ gemm_many_kernel(GemmArgs a) {
       typename W::Scale sc[RT];
 #pragma unroll
       for (int r = 0; r < RT; ++r) {
-        if constexpr (W::kBlocks32)
-          W::template prepare_part<false>(sc[r], raw[r], g);
-        else
-          W::prepare(sc[r], raw[r], g);
+        W::prepare(sc[r], raw[r], g);
+        if constexpr (W::kBlocks32) large |= sc[r].large;
       }
       // the small products have sums of their own where registers allow: each
       // add rounds in proportion to the sum it meets
@@ -745,16 +741,6 @@ gemm_many_kernel(GemmArgs a) {
         hi = *reinterpret_cast<const half8v*>(at);
         lo = *reinterpret_cast<const half8v*>(at + 1024);
       };
-      if constexpr (W::kBlocks32) {
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-          if (__any(sc[r].large)) [[unlikely]]
-            add_part<W, JT, true>(tot[r], raw[r], lane,
-                                  [&](int st, int j, half8v& hi, half8v& lo) { operand(st * JT + j, hi, lo); },
-                                  [&](int j) {
-                                    return *reinterpret_cast<const floatx4*>(buf + L::kInv + 64 * j + 16 * g);
-                                  });
-      }
       half8v ah[2], al[2], bh[RT], bl[RT];
       operand(0, ah[0], al[0]);
 #pragma unroll
@@ -814,6 +800,12 @@ gemm_many_kernel(GemmArgs a) {
     __syncthreads();
   }
 
+  bool anew = false;
+  if constexpr (W::kBlocks32) {
+    anew = __any(large);
+    if (anew) [[unlikely]]
+      sum_in_parts<W, RT, JT>(tot, a, wbase, woff, tok0, kw, KW, lane);
+  }
   if constexpr (KW > 1) {
     floatx4* red = reinterpret_cast<floatx4*>(smem);  // [KW - 1][RW][RT * JT][64]
     if (kw > 0) {
@@ -833,7 +825,7 @@ gemm_many_kernel(GemmArgs a) {
         for (int j = 0; j < JT; ++j)
           tot[r][j] += red[((q * RW + rw) * RT * JT + r * JT + j) * 64 + lane];
   }
-  store_rows(iters > kSegment && KW == 1);
+  store_rows(iters > kSegment && KW == 1 && !anew);
 }
 
 // ---------------------------------------------------------------- F32 rows

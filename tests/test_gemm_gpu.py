@@ -63,6 +63,7 @@ SHAPES = [
     (1, 256, 32, 2), (17, 512, 288, 3), (515, 2048, 1056, 16), (515, 2304, 1856, 17),
     (1024, 2560, 2688, 33), (4096, 256, 544, 31), (4000, 768, 480, 65), (14000, 512, 96, 7),
     (14000, 512, 320, 63), (14000, 256, 256, 130), (14300, 256, 224, 200), (1000, 5120, 4640, 300),
+    (70, 32768, 32736, 20),  # the widest rows
 ]
 
 
@@ -123,7 +124,8 @@ def test_extreme_activations_and_scales(hip, type_tag):
 
 @pytest.mark.parametrize("type_tag", [ggml.Q5_0, ggml.Q8_0], ids=["Q5_0", "Q8_0"])
 @pytest.mark.parametrize("shape", [(40, 480, 3), (515, 1056, 16), (4000, 480, 65), (14000, 320, 63),
-                                   (14300, 256, 200)], ids=lambda s: "x".join(map(str, s)))
+                                   (14300, 256, 200), (14300, 2336, 200)],
+                         ids=lambda s: "x".join(map(str, s)))
 def test_large_scales_leave_small_ones_exact(hip, type_tag, shape):
     """Scales of 256 and more beside scales of 1e-5 to 1e-3: in another row of
     the tile, and in another block of the same row where the large block's
