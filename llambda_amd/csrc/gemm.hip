@@ -66,7 +66,7 @@ struct GemmW<kQ6_K> {
     uint32_t s[2], d;  // scales 8h .. 8h + 7
   };
   struct Scale {
-    half2v sc[4];
+    half2v sc[4];  // 2^-14 sc
   };
   struct Finish {
     float d;
@@ -87,11 +87,11 @@ struct GemmW<kQ6_K> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const uint32_t v = r.s[k >> 1] >> (16 * (k & 1) + b);
-      c.sc[k] = splat2((_Float16)(float)(int)(int8_t)(v & 0xFFu));
+      c.sc[k] = splat2((_Float16)(0x1p-14f * (float)(int)(int8_t)(v & 0xFFu)));
     }
   }
   static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale&, int) {
-    f.d = half_bits_to_float(r.d);
+    f.d = 0x1p14f * half_bits_to_float(r.d);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
                                               int s) {

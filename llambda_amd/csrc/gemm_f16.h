@@ -20,8 +20,9 @@
 //               product: as exact on such tokens, but an activation 2^13 times
 //               the others leaves the rows with the smallest weights for it up
 //               to eight times as far off
-//   Q6_K        sc * (q - 32), 13 bits: hi = the product rounded to f16, lo =
-//               the remainder (exact); d once per chunk
+//   Q6_K        2^-14 sc * (q - 32), 13 bits: hi = the product rounded to f16,
+//               lo = the remainder (exact); 2^14 d once per chunk (d / s alone
+//               would be subnormal in chunks below 2^-99)
 //   Q5_0, Q8_0  d * q, at most 18 bits, as hi + lo (exact: every product is
 //               a multiple of 2^-24, f16's smallest step).  Blocks with a
 //               |d| of 256 or more are multiplied in a part of their own, as

@@ -74,7 +74,7 @@ struct ExpertW<kQ6_K> {
     uint32_t d;
   };
   struct Scale {
-    half2v sc[8];  // scale 2k + (dword >> 2)
+    half2v sc[8];  // 2^-14 times scale 2k + (dword >> 2)
   };
   struct Finish {
     float d;
@@ -98,10 +98,11 @@ struct ExpertW<kQ6_K> {
   static __device__ __forceinline__ void prepare(Scale& c, const Raw& r, int) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      c.sc[i] = splat2((_Float16)(float)(int)(int8_t)(((i < 4 ? r.s.x : r.s.y) >> (8 * (i & 3))) & 0xFFu));
+      c.sc[i] = splat2((_Float16)(
+          0x1p-14f * (float)(int)(int8_t)(((i < 4 ? r.s.x : r.s.y) >> (8 * (i & 3))) & 0xFFu)));
   }
   static __device__ __forceinline__ void finish(Finish& f, const Raw& r, const Scale&, int) {
-    f.d = half_bits_to_float(r.d & 0xFFFFu);
+    f.d = 0x1p14f * half_bits_to_float(r.d & 0xFFFFu);
   }
   static __device__ __forceinline__ void frag(half8v& hi, half8v& lo, const Raw& r, const Scale& c,
                                               int st) {

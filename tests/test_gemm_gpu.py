@@ -191,6 +191,24 @@ def test_one_large_activation(hip, shape):
     assert np.all(err <= bound), float((err / bound).max())
 
 
+@pytest.mark.parametrize("type_tag", TYPES)
+def test_ordinary_scales_at_every_magnitude(hip, type_tag):
+    """Tokens from 1e-36 to 1e34, scales of 1e-4 to 1e-3: neither 1 / s nor its
+    product with a scale may reach the subnormals or overflow."""
+    rows, columns = 160, 1280
+    rng = np.random.default_rng(11)
+    w = synthetic.packed(type_tag, rng, rows, columns)
+    x = synthetic.activations(rng, 24, columns).astype(np.float64)
+    x = (x * 10.0 ** np.linspace(-36, 34, 24)[:, None]).astype(np.float32)
+    s = make_hip_session_packed(w, type_tag, rows, columns)
+    try:
+        for batch in (x, x[:9], x[9:]):  # both kernels
+            _check(type_tag, w, rows, columns, batch, _run(s, np.ascontiguousarray(batch)),
+                   ggml.NAMES[type_tag], norm=False)
+    finally:
+        s.close()
+
+
 @pytest.mark.parametrize("shape", [(1, 4, 2), (33, 260, 16), (515, 1028, 17), (512, 2048, 33),
                                    (96, 4100, 130)], ids=lambda s: "x".join(map(str, s)))
 def test_f32_rows(hip, shape):
