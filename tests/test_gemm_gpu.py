@@ -231,6 +231,30 @@ def test_f32_rows(hip, shape):
     assert np.array_equal(*((first, y[:5]) if tokens > 4 else (again, y[:2])))
 
 
+@pytest.mark.parametrize("shape", [(1, 4, 3), (33, 1028, 4), (515, 4100, 3), (512, 2048, 4), (7, 1020, 2)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_f32_rows_of_two_to_four_tokens(hip, shape):
+    """The kernel of few tokens: tokens and rows short of a workgroup's, columns
+    short of and past a turn of 1024; neighbours of y stay untouched."""
+    import torch
+    rows, columns, tokens = shape
+    rng = np.random.default_rng(rows)
+    w = synthetic.packed(ggml.F32, rng, rows, columns)
+    x = synthetic.activations(rng, tokens, columns)
+    xd = torch.from_numpy(x).cuda()
+    yd = torch.full((tokens * rows + 6,), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    s = make_hip_session_packed(w, ggml.F32, rows, columns)
+    try:
+        s.run_device(xd.data_ptr(), yd[3:].data_ptr(), tokens)
+        torch.cuda.synchronize()
+    finally:
+        s.close()
+    y = yd.cpu().numpy()
+    assert np.all(y[:3] == 7.0) and np.all(y[-3:] == 7.0)
+    _check(ggml.F32, w, rows, columns, x, y[3:-3].reshape(tokens, rows), shape)
+
+
 @pytest.mark.parametrize("type_tag,rows,columns,tokens", [
     (ggml.Q8_0, 16, 32, 16 * 65535 + 20), (ggml.Q5_0, (1 << 20) + 40, 32, 3),
     (ggml.F32, (1 << 20) + 5, 4, 5), (ggml.F32, 7, 8, 16 * 65535 + 9)],

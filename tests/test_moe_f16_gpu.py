@@ -24,7 +24,11 @@ Q4, Q6 = ggml.Q4_K, ggml.Q6_K
     (Q4, Q6, 256, 4, 1, 256, 0, 2), (Q6, Q4, 512, 6, 2, 512, 256, 17),
     (Q4, Q4, 768, 16, 3, 256, 512, 33), (Q6, Q6, 2304, 8, 2, 256, 256, 9),
     (Q4, Q6, 256, 4, 2, 512, 512, 130), (Q4, Q6, 512, 64, 4, 512, 512, 48),
-    (Q4, Q6, 512, 8, 2, 768, 256, 20)])
+    (Q4, Q6, 512, 8, 2, 768, 256, 20),
+    # all of hidden staged at once (few workgroups): 4, 5 and 8 chunks, the last
+    # two against the bits of a batch that stages chunk by chunk
+    (Q6, Q6, 1024, 8, 2, 256, 256, 3), (Q4, Q4, 2048, 8, 2, 256, 0, 2),
+    (Q6, Q4, 1280, 64, 4, 512, 0, 48), (Q4, Q6, 2048, 64, 4, 512, 512, 48)])
 def test_layers(hip, up, down, hidden, experts, top_k, ffn, shared, tokens):
     rng = np.random.default_rng(hidden + tokens)
     layer = synthetic_qwen3next(rng, hidden=hidden, experts=experts, top_k=top_k, ffn=ffn,
