@@ -28,9 +28,9 @@ gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
   extern __shared__ float smem[];
   float* xs = smem;
   float* xg = smem + K;
-  stage_x<1>(xs, xg, x, K, 1, K);
+  stage_x(xs, xg, x, K);
   __syncthreads();
-  const XView xv{xs, xg, K, K >> 4};
+  const XView xv{xs, xg};
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -44,7 +44,7 @@ gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
   const int stride = gridDim.x * waves_per_block * rows_per_iter;
 
   for (int base = (blockIdx.x * waves_per_block + wave) * rows_per_iter; base < rows; base += stride) {
-    float acc[R][1];
+    float acc[R];
     const uint8_t* rp[R];
     bool valid[R];
 #pragma unroll
@@ -53,11 +53,11 @@ gemv_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, int rows, int K,
       valid[r] = row < rows;
       rp[r] = w + (int64_t)(valid[r] ? row : 0) * row_bytes;
     }
-    rows_dot<TYPE, 1, R>(rp, valid, l, lpr, units, xv, acc);
+    rows_dot<TYPE, R>(rp, valid, l, lpr, units, xv, acc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int row = base + r * slots + slot;
-      const float v = segment_sum_dyn(acc[r][0], lpr);
+      const float v = segment_sum_dyn(acc[r], lpr);
       if (l == 0 && row < rows) y[row] = v;
     }
   }

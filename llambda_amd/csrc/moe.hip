@@ -418,13 +418,9 @@ hipError_t moe_forward_launch(const MoePlan& p, const float* x, float* y, int to
     a.expert_stride = p.up_g_stride;
     a.s_w0 = p.sh_up_g;
   }
-  if (f16)
-    e = moe_f16_up_launch(p.up_type, a, mt, routed_chunks + (joint_up ? shared_chunks : 0), s);
-  else
-  e = moe_gemm_launch(p.up_type, epi, a, mt,
-                      fuse_gate ? K + (joint_up ? 1 : 0)
-                                : routed_chunks + (joint_up ? shared_chunks : 0),
-                      s);
+  const int up_chunks = routed_chunks + (joint_up ? shared_chunks : 0);
+  e = f16 ? moe_f16_up_launch(p.up_type, a, mt, up_chunks, s)
+          : moe_gemm_launch(p.up_type, epi, a, mt, fuse_gate ? K + (joint_up ? 1 : 0) : up_chunks, s);
   if (e != hipSuccess) return e;
   if (has_shared && !joint_up) {
     a = up;

@@ -26,13 +26,10 @@
 
 namespace llhip {
 
-// x for NT tokens lives in LDS as xs[tok * xs_stride + k] and the sums of
-// its 16-element groups as xg[tok * xg_stride + k/16].
+// x lives in LDS as xs[k] and the sums of its 16-element groups as xg[k / 16].
 struct XView {
   const float* xs;
   const float* xg;
-  int xs_stride;
-  int xg_stride;
 };
 
 template <int TYPE>
@@ -69,8 +66,7 @@ struct Unit<kQ4_K> {
       m = (int)((B8 >> 4) | ((B4 >> 6) << 4));
     }
   }
-  template <int NT>
-  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float (&acc)[NT]) {
+  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float& acc) {
     const int t = unit & 7, j = t >> 1, half = t & 1;
     int sc0, m0, sc1, m1;
     scale_min(r.hdr, 2 * j, sc0, m0);
@@ -93,33 +89,30 @@ struct Unit<kQ4_K> {
     }
     const int xl = (unit >> 3) * 256 + 64 * j + 16 * half;
     const int xh = xl + 32;
+    const float4* pl = reinterpret_cast<const float4*>(xv.xs + xl);
+    const float4* ph = reinterpret_cast<const float4*>(xv.xs + xh);
+    float al = 0.f, ah = 0.f;
 #pragma unroll
-    for (int tok = 0; tok < NT; ++tok) {
-      const float4* pl = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + xl);
-      const float4* ph = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + xh);
-      float al = 0.f, ah = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        float4 a = pl[w];
-        float4 b = ph[w];
-        al = fmaf(wl[4 * w + 0], a.x, al);
-        al = fmaf(wl[4 * w + 1], a.y, al);
-        al = fmaf(wl[4 * w + 2], a.z, al);
-        al = fmaf(wl[4 * w + 3], a.w, al);
-        ah = fmaf(wh[4 * w + 0], b.x, ah);
-        ah = fmaf(wh[4 * w + 1], b.y, ah);
-        ah = fmaf(wh[4 * w + 2], b.z, ah);
-        ah = fmaf(wh[4 * w + 3], b.w, ah);
-      }
-      const float gl = xv.xg[tok * xv.xg_stride + (xl >> 4)];
-      const float gh = xv.xg[tok * xv.xg_stride + (xh >> 4)];
-      float v = acc[tok];
-      v = fmaf(delta0, al, v);
-      v = fmaf(-off0, gl, v);
-      v = fmaf(delta1, ah, v);
-      v = fmaf(-off1, gh, v);
-      acc[tok] = v;
+    for (int w = 0; w < 4; ++w) {
+      float4 a = pl[w];
+      float4 b = ph[w];
+      al = fmaf(wl[4 * w + 0], a.x, al);
+      al = fmaf(wl[4 * w + 1], a.y, al);
+      al = fmaf(wl[4 * w + 2], a.z, al);
+      al = fmaf(wl[4 * w + 3], a.w, al);
+      ah = fmaf(wh[4 * w + 0], b.x, ah);
+      ah = fmaf(wh[4 * w + 1], b.y, ah);
+      ah = fmaf(wh[4 * w + 2], b.z, ah);
+      ah = fmaf(wh[4 * w + 3], b.w, ah);
     }
+    const float gl = xv.xg[xl >> 4];
+    const float gh = xv.xg[xh >> 4];
+    float v = acc;
+    v = fmaf(delta0, al, v);
+    v = fmaf(-off0, gl, v);
+    v = fmaf(delta1, ah, v);
+    v = fmaf(-off1, gh, v);
+    acc = v;
   }
 };
 
@@ -154,8 +147,7 @@ struct Unit<kQ6_K> {
     uint32_t w = (i < 4) ? sc.x : (i < 8) ? sc.y : (i < 12) ? sc.z : sc.w;
     return (int)(int8_t)((w >> (8 * (i & 3))) & 0xFFu);
   }
-  template <int NT>
-  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float (&acc)[NT]) {
+  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float& acc) {
     const int t = unit & 7, h = t >> 2, part = (t >> 1) & 1, half = t & 1;
     const float d = half_bits_to_float(r.dword & 0xFFFFu);
     const int ia = 8 * h + half + 2 * part;  // scale of q_k, k = part
@@ -177,31 +169,28 @@ struct Unit<kQ6_K> {
     }
     const int xa = (unit >> 3) * 256 + 128 * h + 32 * part + 16 * half;
     const int xb = xa + 64;
+    const float4* pa = reinterpret_cast<const float4*>(xv.xs + xa);
+    const float4* pb = reinterpret_cast<const float4*>(xv.xs + xb);
+    float sa_ = 0.f, sb_ = 0.f;
 #pragma unroll
-    for (int tok = 0; tok < NT; ++tok) {
-      const float4* pa = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + xa);
-      const float4* pb = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + xb);
-      float sa_ = 0.f, sb_ = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        float4 a = pa[w];
-        float4 b = pb[w];
-        sa_ = fmaf(wa[4 * w + 0], a.x, sa_);
-        sa_ = fmaf(wa[4 * w + 1], a.y, sa_);
-        sa_ = fmaf(wa[4 * w + 2], a.z, sa_);
-        sa_ = fmaf(wa[4 * w + 3], a.w, sa_);
-        sb_ = fmaf(wb[4 * w + 0], b.x, sb_);
-        sb_ = fmaf(wb[4 * w + 1], b.y, sb_);
-        sb_ = fmaf(wb[4 * w + 2], b.z, sb_);
-        sb_ = fmaf(wb[4 * w + 3], b.w, sb_);
-      }
-      const float ga = xv.xg[tok * xv.xg_stride + (xa >> 4)];
-      const float gb = xv.xg[tok * xv.xg_stride + (xb >> 4)];
-      float v = acc[tok];
-      v = fmaf(delta_a, fmaf(-32.f, ga, sa_), v);
-      v = fmaf(delta_b, fmaf(-32.f, gb, sb_), v);
-      acc[tok] = v;
+    for (int w = 0; w < 4; ++w) {
+      float4 a = pa[w];
+      float4 b = pb[w];
+      sa_ = fmaf(wa[4 * w + 0], a.x, sa_);
+      sa_ = fmaf(wa[4 * w + 1], a.y, sa_);
+      sa_ = fmaf(wa[4 * w + 2], a.z, sa_);
+      sa_ = fmaf(wa[4 * w + 3], a.w, sa_);
+      sb_ = fmaf(wb[4 * w + 0], b.x, sb_);
+      sb_ = fmaf(wb[4 * w + 1], b.y, sb_);
+      sb_ = fmaf(wb[4 * w + 2], b.z, sb_);
+      sb_ = fmaf(wb[4 * w + 3], b.w, sb_);
     }
+    const float ga = xv.xg[xa >> 4];
+    const float gb = xv.xg[xb >> 4];
+    float v = acc;
+    v = fmaf(delta_a, fmaf(-32.f, ga, sa_), v);
+    v = fmaf(delta_b, fmaf(-32.f, gb, sb_), v);
+    acc = v;
   }
 };
 
@@ -229,8 +218,7 @@ struct Unit<kQ8_0> {
     load_dwords_unaligned2<9>(row + unit * 34, r.w);
     return r;
   }
-  template <int NT>
-  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float (&acc)[NT]) {
+  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float& acc) {
     const float d = half_bits_to_float(r.w[0] & 0xFFFFu);
     float u[32];
 #pragma unroll
@@ -241,21 +229,18 @@ struct Unit<kQ8_0> {
       for (int k = 0; k < 4; ++k) u[4 * w + k] = ubyte(v, k);
     }
     const int x0 = unit * 32;
+    const float4* p = reinterpret_cast<const float4*>(xv.xs + x0);
+    float s = 0.f;
 #pragma unroll
-    for (int tok = 0; tok < NT; ++tok) {
-      const float4* p = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + x0);
-      float s = 0.f;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        float4 a = p[w];
-        s = fmaf(u[4 * w + 0], a.x, s);
-        s = fmaf(u[4 * w + 1], a.y, s);
-        s = fmaf(u[4 * w + 2], a.z, s);
-        s = fmaf(u[4 * w + 3], a.w, s);
-      }
-      const float g = xv.xg[tok * xv.xg_stride + 2 * unit] + xv.xg[tok * xv.xg_stride + 2 * unit + 1];
-      acc[tok] = fmaf(d, fmaf(-128.f, g, s), acc[tok]);
+    for (int w = 0; w < 8; ++w) {
+      float4 a = p[w];
+      s = fmaf(u[4 * w + 0], a.x, s);
+      s = fmaf(u[4 * w + 1], a.y, s);
+      s = fmaf(u[4 * w + 2], a.z, s);
+      s = fmaf(u[4 * w + 3], a.w, s);
     }
+    const float g = xv.xg[2 * unit] + xv.xg[2 * unit + 1];
+    acc = fmaf(d, fmaf(-128.f, g, s), acc);
   }
 };
 
@@ -274,8 +259,7 @@ struct Unit<kQ5_0> {
   static __device__ __forceinline__ uint32_t spread4(uint32_t nib) {
     return ((nib * 0x00204081u) & 0x01010101u) << 4;
   }
-  template <int NT>
-  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float (&acc)[NT]) {
+  static __device__ __forceinline__ void dot(const Raw& r, int unit, const XView& xv, float& acc) {
     const float d = half_bits_to_float(r.w[0] & 0xFFFFu);
     const uint32_t qh = __builtin_amdgcn_alignbyte(r.w[1], r.w[0], 2);
     float ul[16], uh[16];
@@ -292,68 +276,50 @@ struct Unit<kQ5_0> {
       }
     }
     const int x0 = unit * 32;
+    const float4* p = reinterpret_cast<const float4*>(xv.xs + x0);
+    float s = 0.f;
 #pragma unroll
-    for (int tok = 0; tok < NT; ++tok) {
-      const float4* p = reinterpret_cast<const float4*>(xv.xs + tok * xv.xs_stride + x0);
-      float s = 0.f;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        float4 a = p[w];
-        float4 b = p[4 + w];
-        s = fmaf(ul[4 * w + 0], a.x, s);
-        s = fmaf(ul[4 * w + 1], a.y, s);
-        s = fmaf(ul[4 * w + 2], a.z, s);
-        s = fmaf(ul[4 * w + 3], a.w, s);
-        s = fmaf(uh[4 * w + 0], b.x, s);
-        s = fmaf(uh[4 * w + 1], b.y, s);
-        s = fmaf(uh[4 * w + 2], b.z, s);
-        s = fmaf(uh[4 * w + 3], b.w, s);
-      }
-      const float g = xv.xg[tok * xv.xg_stride + 2 * unit] + xv.xg[tok * xv.xg_stride + 2 * unit + 1];
-      acc[tok] = fmaf(d, fmaf(-16.f, g, s), acc[tok]);
+    for (int w = 0; w < 4; ++w) {
+      float4 a = p[w];
+      float4 b = p[4 + w];
+      s = fmaf(ul[4 * w + 0], a.x, s);
+      s = fmaf(ul[4 * w + 1], a.y, s);
+      s = fmaf(ul[4 * w + 2], a.z, s);
+      s = fmaf(ul[4 * w + 3], a.w, s);
+      s = fmaf(uh[4 * w + 0], b.x, s);
+      s = fmaf(uh[4 * w + 1], b.y, s);
+      s = fmaf(uh[4 * w + 2], b.z, s);
+      s = fmaf(uh[4 * w + 3], b.w, s);
     }
+    const float g = xv.xg[2 * unit] + xv.xg[2 * unit + 1];
+    acc = fmaf(d, fmaf(-16.f, g, s), acc);
   }
 };
 
 // ------------------------------------------------------------------ staging
-// Copy NT activation rows into LDS (rows with a null source become zero) and
-// form the sums of each 16-element group.  Four consecutive threads stage one
-// group, so the group sum is two shuffles.  K must be a multiple of 32.
-template <int NT>
-__device__ __forceinline__ void stage_rows(float* xs, float* xg, const float* const* src, int K) {
+// Copy the activations into LDS and form the sums of each 16-element group.
+// Four consecutive threads stage one group, so the group sum is two shuffles.
+// K must be a multiple of 32.
+__device__ __forceinline__ void stage_x(float* xs, float* xg, const float* __restrict__ x, int K) {
   const int n4 = K >> 2;
-  const int total = NT * n4;
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int tok = i / n4, k4 = i - tok * n4;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (src[tok]) v = reinterpret_cast<const float4*>(src[tok])[k4];
-    reinterpret_cast<float4*>(xs + tok * K)[k4] = v;
+  for (int k4 = threadIdx.x; k4 < n4; k4 += blockDim.x) {
+    const float4 v = reinterpret_cast<const float4*>(x)[k4];
+    reinterpret_cast<float4*>(xs)[k4] = v;
     float s = (v.x + v.y) + (v.z + v.w);
     s += __shfl_xor(s, 1, kWave);
     s += __shfl_xor(s, 2, kWave);
-    if ((k4 & 3) == 0) xg[tok * (K >> 4) + (k4 >> 2)] = s;
+    if ((k4 & 3) == 0) xg[k4 >> 2] = s;
   }
 }
 
-template <int NT>
-__device__ __forceinline__ void stage_x(float* xs, float* xg, const float* __restrict__ x,
-                                        int64_t x_stride, int ntok, int K) {
-  const float* src[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) src[t] = t < ntok ? x + t * x_stride : nullptr;
-  stage_rows<NT>(xs, xg, src, K);
-}
-
-// Dot of R packed rows (row pointers rp) with NT staged activations: lane l of
+// Dot of R packed rows (row pointers rp) with the staged activations: lane l of
 // a `lpr`-lane slot covers units l, l + lpr, ...; the caller sums the slot.
-template <int TYPE, int NT, int R>
+template <int TYPE, int R>
 __device__ __forceinline__ void rows_dot(const uint8_t* const (&rp)[R], const bool (&valid)[R],
                                          int l, int lpr, int units, const XView& xv,
-                                         float (&acc)[R][NT]) {
+                                         float (&acc)[R]) {
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[r][t] = 0.f;
+  for (int r = 0; r < R; ++r) acc[r] = 0.f;
   for (int u0 = 0; u0 < units; u0 += lpr) {
     const int u = u0 + l;
     typename Unit<TYPE>::Raw raw[R];
@@ -365,7 +331,7 @@ __device__ __forceinline__ void rows_dot(const uint8_t* const (&rp)[R], const bo
     }
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      if (ok[r]) Unit<TYPE>::template dot<NT>(raw[r], u, xv, acc[r]);
+      if (ok[r]) Unit<TYPE>::dot(raw[r], u, xv, acc[r]);
   }
 }
 
