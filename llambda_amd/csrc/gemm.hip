@@ -447,13 +447,16 @@ gemm_few_kernel(GemmArgs a) {
         blk = mfma_f16(al[st], bh[st], blk);
         if constexpr (W::kPair) blk = mfma_f16(ah[st], bl, blk);
       }
-#pragma unroll
-      for (int st = 0; st < (W::kMin ? 4 : 8); ++st) blk = mfma_f16(ah[st], bh[st], blk);
       if constexpr (W::kMin) {
-        floatx4 half = {0.f, 0.f, 0.f, 0.f};
+        // in quarters: their chains run side by side
+        floatx4 part[4];
 #pragma unroll
-        for (int st = 4; st < 8; ++st) half = mfma_f16(ah[st], bh[st], half);
-        blk += half;
+        for (int st = 0; st < 8; ++st)
+          part[st >> 1] = mfma_f16(ah[st], bh[st], st & 1 ? part[st >> 1] : floatx4{0.f, 0.f, 0.f, 0.f});
+        blk += (part[0] + part[1]) + (part[2] + part[3]);
+      } else {
+#pragma unroll
+        for (int st = 0; st < 8; ++st) blk = mfma_f16(ah[st], bh[st], blk);
       }
       typename W::Finish fin;
       W::finish(fin, raw[r], sc, g);
