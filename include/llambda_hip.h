@@ -107,7 +107,8 @@ int llambda_hip_session_run(llambda_hip_session* session, const float* input,
 
 /* Multi-token form: input [batch][K], output [batch][N], synchronous.  No
  * counterpart in the reference (its prefill is one token at a time,
- * llambda.lisp:1319-1341); row t equals session_run on row t. */
+ * llambda.lisp:1319-1341); row t equals session_run on row t to the rounding
+ * of single floats (the order of a row's sums follows the batch). */
 int llambda_hip_session_run_batch(llambda_hip_session* session, const float* input,
                                   size_t input_element_count, float* output,
                                   size_t output_element_count, size_t batch);
@@ -115,7 +116,8 @@ int llambda_hip_session_run_batch(llambda_hip_session* session, const float* inp
 /* Device-resident form: input/output are device pointers ([batch][K],
  * [batch][N]); the kernels are enqueued on `stream` (a hipStream_t, or null
  * for the session's own stream) and the call returns without waiting.
- * For callers that keep activations in HBM (and for benchmarking). */
+ * For callers that keep activations in HBM (and for benchmarking).  Batches of
+ * two or more may keep partial sums in `output` until the last kernel ends. */
 int llambda_hip_session_run_device(llambda_hip_session* session, const float* input,
                                    float* output, size_t batch, void* stream);
 

@@ -350,9 +350,11 @@ __device__ __forceinline__ void sum_in_parts(floatx4 (&tot)[RT][JT], const GemmA
 // 16 RT rows and deal the chunks among themselves, each wave holding its
 // chunk's activations in registers (lane (t, g) loads, scales and splits the
 // 64 elements its own operand slots need: no LDS, no barrier before the
-// waves' sums meet).  Bound by reading the weights once and by unpacking them:
-// 7 tokens through Q4_K 14336 x 4096 take 15.0 us (2.2 TB/s; 186 us when each
-// four tokens read the rows again and the VALU formed the products).
+// waves' sums meet).  7 tokens through Q4_K 14336 x 4096 take 14.9 us (2.2
+// TB/s; 186 us when each four tokens read the rows again and the VALU formed
+// the products).  There the VALU issues for 40% of the SIMD cycles (splitting
+// x and unpacking) and the matrix cores work for 11%; the rest is latency:
+// nothing of a wave's next chunk is requested before this one is done.
 template <int TYPE, int RT, int KW>
 __global__ void __launch_bounds__(64 * KW)
 gemm_few_kernel(GemmArgs a) {
@@ -523,12 +525,13 @@ __device__ __forceinline__ float scatter_sum(const float* v, bool b2, bool b1, b
 // 16 lanes, and the operand image is [token tile][step][hi, lo][16 bytes per
 // lane], lane positions XORed with the step so that the writes of one
 // instruction spread over the banks.
-// Measured: 2048 tokens through Q4_K 14336 x 4096 0.67 ms (360 TFLOP/s; 49.8
-// ms before, in passes of four tokens on the VALU), 1000 tokens through Q6_K
-// 4096 x 14336 0.41 ms (31.7), 129 through Q8_0 1024 x 2688 14.9 us (517).
-// Bound by the VALU beside the MFMAs (unpacking and splitting: about four
-// instructions per MFMA, two of which issue beside it) and the operand reads
-// (a wave of 32 rows reads each split activation once per 32 rows).
+// Measured, card to card: 2048 tokens through Q4_K 14336 x 4096 0.63 to 0.70 ms
+// (340 to 380 TFLOP/s; 49.8 ms in passes of four tokens on the VALU), 1000
+// tokens through Q6_K 4096 x 14336 0.40 to 0.45 ms (31.7), 129 through Q8_0
+// 1024 x 2688 14.6 us (517).  Bound by
+// instruction issue: of the SIMD cycles of the first the VALU takes 47% (5.4
+// instructions per MFMA: unpacking, splitting, adding the chunks' sums) and
+// the matrix cores 35, of the second 38 and 38.
 template <int TYPE, int JT>
 struct GemmLds {
   static constexpr int kX = JT * 16384;             // split activations
@@ -704,8 +707,8 @@ gemm_many_kernel(GemmArgs a) {
     }
     each([&](float& v, int r, int j, int i) { v = tot[r][j][i]; });
   };
-  // One group's totals go out every 8 chunks and start again: each add to them
-  // rounds in proportion to what they have reached (16 chunks of Q4_K in one
+  // One group's totals go out to y every 8 chunks, where the next ones are added
+  // to them, and start again: each add to them rounds in proportion to what they have reached (16 chunks of Q4_K in one
   // run: 1.24e-7 against 64 bits, an fp32 evaluation 1.17e-7)
   constexpr int kSegment = 8;
 
@@ -838,8 +841,8 @@ gemm_many_kernel(GemmArgs a) {
 // bytes a row).  Each token's sums run in one
 // order whatever the batch and JT.  Bound by the loads' latency at few tokens
 // (512 x 2048, 7 tokens: 19.8 -> 11.7 us), by the fp32 MFMA at many (2048 x
-// 4096, 512 tokens: 3.6 ms in passes of four tokens on the VALU -> 0.123 ms,
-// 70 of 157 TFLOP/s); errors against 64 bits 0.8e-7 to 1.0e-7 (0.8e-7 to
+// 4096, 512 tokens: 3.6 ms in passes of four tokens on the VALU -> 0.12 to
+// 0.14 ms, 63 to 70 of 157 TFLOP/s); errors against 64 bits 0.8e-7 to 1.0e-7 (0.8e-7 to
 // 1.6e-7 before).
 constexpr int kF32Waves = 8;
 template <int JT>
@@ -1021,10 +1024,14 @@ static hipError_t launch_type(const GemmArgs& a, bool one_order, hipStream_t str
   if (one_order) return launch_many<TYPE, 2, 1, 2, 4>(a, stream);
   // The tile shape whose workgroups, one to a CU, finish first: rounds of
   // workgroups times a workgroup's time, in 0.1 us for 16 chunks of Q4_K
-  // (measured with one round; the other types' times stand in the same
-  // proportions).  Small tiles leave fewer CUs idle, large ones decode and
-  // split less per product: 256 x 64 does 172 rows x tokens a us, 128 x 32
-  // 117, 32 x 16 40.
+  // (measured with one round).  Small tiles leave fewer CUs idle, large ones
+  // decode and split less per product: 256 x 64 does 172 rows x tokens a us,
+  // 128 x 32 117, 32 x 16 40.  With other chunk counts and types only the
+  // proportions matter: of 70 calls (Q4_K of 2, 16 and 56 chunks, Q6_K of 16
+  // and 56, Q8_0 of 11, Q5_0 of 4; 1024 to 14336 rows, 4 to 500 tokens) the
+  // shape taken was within 3% of the fastest of the eight in 63, and 6 to 24%
+  // off where rows are short or three token tiles of a pair type meet 64 row
+  // tiles (Q4_K 14336 x 512, 7 tokens: 5.6 us, 4.5 in 64 x 16 tiles of many).
   struct Shape {
     int rows, tokens, base, per_token;  // per_token: of the first 16 tokens
   };

@@ -24,8 +24,12 @@
 
 namespace llhip {
 
-constexpr int kWaves = 8;      // per workgroup: two workgroups per CU
-constexpr int kDownChunks = 2; // chunks of the down products' K held in LDS
+constexpr int kWaves = 8;  // per workgroup: two workgroups per CU
+// Chunks of the down products' K held in LDS: two (ffn 512, the Qwen3Next
+// layers') leave two workgroups to a CU at two token tiles (70 KB).  Four would
+// fit (139 KB, one workgroup); wider ffn keep the bf16 pipelines, unmeasured
+// here.
+constexpr int kDownChunks = 2;
 
 // ------------------------------------------------------------- products
 // Activations reach the products through LDS: one operand (a step's hi or lo
@@ -142,10 +146,11 @@ __device__ __forceinline__ int entry_pair(const MoeGemmArgs& a, const MoeChunk& 
 // same order; 2 tokens of a Qwen3Next layer: 63 -> 47 us with the down launch's
 // shorter workgroups; from 344 workgroups on the two that share a CU win: 8
 // tokens 83 us deep, 76 not, 256 tokens 352 and 315).
-// Measured for 256 tokens (E 512, top 10, 634 MB of rows): 156 us, 4.1 TB/s
-// (177 us with bf16 parts, whose group sums the VALU scaled; 180 us as one
+// Measured for 256 tokens (E 512, top 10, 634 MB of rows): 153 to 163 us, 4.0
+// TB/s (177 us with bf16 parts, whose group sums the VALU scaled; 180 us as one
 // workgroup of 16 waves per CU, whose start, end and waits nothing covered).
-// Bound by the rows' round trips behind the barriers.
+// The VALU issues for 53% of the SIMD cycles (9.4 instructions per MFMA: most
+// experts have 5 pairs of the tile's 16) and the matrix cores work for 23.
 template <int TYPE, int JT, bool DEEP>
 __global__ void __launch_bounds__(64 * kWaves, JT == 1 && !DEEP ? 4 : 2)
 expert_up_kernel(MoeGemmArgs a) {
@@ -240,8 +245,8 @@ expert_up_kernel(MoeGemmArgs a) {
 // Down rows, fp32 outputs per pair: a workgroup forms its entry's images once
 // (K of at most kDownChunks chunks), then its waves take two row tiles at a
 // time over all of K, the rows of the next step always in flight.  256 tokens
-// as above (457 MB of rows): 122 us (174 us with bf16 parts in 16-wide
-// products).
+// as above (457 MB of rows): 125 to 132 us (174 us with bf16 parts in 16-wide
+// products); VALU 51% of the SIMD cycles, matrix cores 19.
 template <int TYPE, int JT>
 __global__ void __launch_bounds__(64 * kWaves, JT == 1 ? 4 : 2)
 expert_down_kernel(MoeGemmArgs a) {
