@@ -360,7 +360,8 @@ __global__ void __launch_bounds__(64 * KW)
 gemm_few_kernel(GemmArgs a) {
   using W = GemmW<TYPE>;
   __shared__ floatx4 red[KW > 1 ? KW - 1 : 1][RT][64];
-  const int lane = threadIdx.x & 63, kw = threadIdx.x >> 6;
+  // the wave's number is uniform: so are the loop over its chunks and their bases
+  const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g = lane >> 4;
   const int row0 = blockIdx.x * 16 * RT, tok0 = blockIdx.y * 16;
   const float* xr = a.x + (int64_t)min(tok0 + n, a.tokens - 1) * a.x_stride;
